@@ -304,13 +304,6 @@ __device__ __forceinline__ int64_t frag_block(int w0, int i, int pairs, int pair
     return ((int64_t)(w0 + i) * 2 + (i == 0 ? 1 : 0)) * pairs + pair;
 }
 
-// Log-sum-exp merge of the fragments (ranges w0..w1) of sequence s for one
-// wave's heads head_base .. head_base+gc-1.  Each chunk of 8 fragments is one
-// round of loads: every (m, l) and every partial output of the chunk is
-// requested before any is used, then folded in with an online rescale.
-// Lane (i8, h) = (lane / 8, lane % 8) owns fragment weights; output element
-// e = lane + 64 k (head e / D) of the 8 x D block is lane-owned.  `wts` is the
-// wave's LDS scratch (>= 80 floats).
 // Workgroup spans of the split axis (Tv tiles, G ranges walked by WG
 // workgroups, WG <= G): workgroup w covers ranges [range_start(w, G, WG),
 // range_start(w + 1, G, WG)).  With WG == G a span is one range.
@@ -353,77 +346,75 @@ struct Spans {
     __device__ bool live(int w) const { return sp.all_live() || start(w) < start(w + 1); }
 };
 
-template <int D>
-__device__ __forceinline__ void merge_fragments(const DecodeParams& p, int s, int w0, int w1,
-                                                int pair, int head_base, int gc, const Spans& sp,
-                                                int lane,
-                                                __attribute__((address_space(3))) float* wts) {
-    // output element e = 4 lane + 256 k4 (.. +3, all in head e / D since D % 4 == 0)
-    constexpr int K4 = (8 * D + 255) / 256;
-    const int nfr = w1 - w0 + 1;
-    const int i8 = lane >> 3, h = lane & 7;
-    const int n_out = gc * D;
-    const auto mlr = make_rsrc(p.ws_ml, 0x7FFFFFFF);
-    float M = kMaxSeed, L = 0.f;  // of head h
-    f4 acc[K4];
+// Log-sum-exp merge of one lane's 4 output elements over nfr fragments.
+// The FW waves of a unit take the fragments in chunks of 8 (wave fw: chunks
+// fw, fw + FW, ..): one round of loads per chunk, every (m, l) and partial
+// output requested before any is used, then folded in with an online rescale;
+// each lane reads its own head's (m, l), so a chunk needs no cross-lane step.
+// The waves' partials meet in LDS and wave 0 of the unit writes.
+//
+// What bounds it is the chain of rounds (about 1 us each), not bytes: one
+// wave per 8 heads folding the 256 fragments of one 32768-token sequence took
+// 62 us of its decode, 8 waves per 256 outputs take 8 (merge_waves).
+//   ok(i)      fragment i holds tokens (fragment 0 always does)
+//   ml(i)      address of its (m, l) for this lane's head
+//   o(i)       address of this lane's 4 outputs in it
+constexpr int kMergeChunk = 8;
+
+template <int FW, class Ok, class Ml, class O>
+__device__ __forceinline__ void merge_unit(int nfr, int fw, int lane, bool act, float* out, Ok ok, Ml ml, O o,
+                                           float (*lds)[64][6]) {
+    float M = kMaxSeed, L = 0.f;
+    f4 acc = {0.f, 0.f, 0.f, 0.f};
+    for (int i0 = fw * kMergeChunk; i0 < nfr; i0 += FW * kMergeChunk) {
+        float2 x[kMergeChunk];
+        f4 v[kMergeChunk];
+        bool live[kMergeChunk];
 #pragma unroll
-    for (int k = 0; k < K4; ++k) acc[k] = f4{0.f, 0.f, 0.f, 0.f};
-    for (int i0 = 0; i0 < nfr; i0 += 8) {
-        // one round of loads for the chunk
-        float2 ml = make_float2(kMaxSeed, 0.f);
-        {
-            const int i = i0 + i8;
-            const bool ok = i < nfr && h < gc && sp.live(w0 + i);
-            const int64_t idx = frag_block(w0, ok ? i : 0, p.pairs, pair) * 16 + h;
-            const float2 x = __builtin_bit_cast(
-                float2, __builtin_amdgcn_raw_buffer_load_b64(mlr, (int)(idx * 8), 0, 0));
-            if (ok) ml = x;
+        for (int j = 0; j < kMergeChunk; ++j) {
+            live[j] = i0 + j < nfr && ok(i0 + j);
+            const int i = live[j] ? i0 + j : 0;  // a missing fragment reads fragment 0, weight 0 below
+            x[j] = *ml(i);
+            v[j] = *reinterpret_cast<const f4*>(o(i));
         }
-        f4 v[8][K4];
+        float Mn = M;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            // an empty or missing fragment reads fragment 0 (weight 0 below)
-            const int i = i0 + j;
-            const bool ok = i < nfr && sp.live(w0 + i);
-            const float* row = p.ws_o + frag_block(w0, ok ? i : 0, p.pairs, pair) * (8 * D);
-            const auto rr = make_rsrc(row, n_out * 4);
-#pragma unroll
-            for (int k = 0; k < K4; ++k)
-                v[j][k] = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(
-                                                     rr, (4 * lane + 256 * k) * 4, 0, 0));
-        }
-        // running max / sum of head h, chunk weights
-        float cm = ml.x;
-        cm = fmaxf(cm, __shfl_xor(cm, 8, 64));
-        cm = fmaxf(cm, __shfl_xor(cm, 16, 64));
-        cm = fmaxf(cm, __shfl_xor(cm, 32, 64));
-        const float Mn = fmaxf(M, cm);
-        const float wt = fast_exp2(ml.x - Mn);  // 0 for empty fragments
-        float cl = wt * ml.y;
-        cl += __shfl_xor(cl, 8, 64);
-        cl += __shfl_xor(cl, 16, 64);
-        cl += __shfl_xor(cl, 32, 64);
-        const float resc = fast_exp2(M - Mn);
-        L = L * resc + cl;
+        for (int j = 0; j < kMergeChunk; ++j) Mn = fmaxf(Mn, live[j] ? x[j].x : kMaxSeed);
+        const float r = fast_exp2(M - Mn);
+        L *= r;
+        acc *= r;
         M = Mn;
-        wts[lane] = wt;                       // wts[i8 * 8 + h]
-        if (lane < 8) wts[64 + lane] = resc;  // rescale of head `lane`
 #pragma unroll
-        for (int k = 0; k < K4; ++k) {
-            const int hk = min((4 * lane + 256 * k) / D, 7);
-            f4 a = acc[k] * wts[64 + hk];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) a += wts[j * 8 + hk] * v[j][k];
-            acc[k] = a;
+        for (int j = 0; j < kMergeChunk; ++j) {
+            const float w = live[j] ? fast_exp2(x[j].x - Mn) : 0.f;
+            L += w * x[j].y;
+            acc += w * v[j];
         }
     }
-    if (lane < 8) wts[72 + lane] = 1.0f / (L + 1e-9f);
-    float* out = p.out + ((int64_t)s * p.num_heads + head_base) * D;
+    if constexpr (FW > 1) {
+        float* e = lds[fw][lane];
+        e[0] = M;
+        e[1] = L;
 #pragma unroll
-    for (int k = 0; k < K4; ++k) {
-        const int e = 4 * lane + 256 * k;
-        if (e < n_out) *reinterpret_cast<f4*>(out + e) = acc[k] * wts[72 + e / D];
+        for (int k = 0; k < 4; ++k) e[2 + k] = acc[k];
+        __syncthreads();
+        if (fw > 0) return;
+        float Mn = M;
+#pragma unroll
+        for (int w = 1; w < FW; ++w) Mn = fmaxf(Mn, lds[w][lane][0]);
+        const float r = fast_exp2(M - Mn);
+        L *= r;
+        acc *= r;
+#pragma unroll
+        for (int w = 1; w < FW; ++w) {
+            const float* y = lds[w][lane];
+            const float wt = fast_exp2(y[0] - Mn);  // 0 for a wave without fragments
+            L += wt * y[1];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) acc[k] += wt * y[2 + k];
+        }
     }
+    if (act) *reinterpret_cast<f4*>(out) = acc * (1.0f / (L + 1e-9f));
 }
 
 template <int KV, int D, int TPS, int NBUF>
@@ -699,24 +690,35 @@ void decode_mfma_kernel(DecodeParams p) {
     }
 }
 
-// One wave per (sequence, kv-head slot): sequences split over several ranges
-// get their partial blocks merged; everything else was finished in place.
-template <int D>
-__global__ __launch_bounds__(256) void merge_split_kernel(DecodeParams p) {
-    __shared__ float wts_all[4][80];
+// Sequences split over several ranges get their partial blocks merged;
+// everything else was finished in place.  A unit of work is 256 outputs of
+// one (sequence, kv-head slot): grid (sequence, 4 slots, slot of the 4 and
+// units / SL), SL units of FW waves per workgroup.
+template <int D, int SL, int FW>
+__global__ __launch_bounds__(SL * FW * 64) void merge_split_kernel(DecodeParams p) {
+    __shared__ float part[FW > 1 ? SL * FW : 1][64][6];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int pair = blockIdx.y * 4 + wave;
+    const int fw = wave % FW, sl = wave / FW;
+    const int pair = 4 * blockIdx.y + (blockIdx.z & 3), unit = (blockIdx.z >> 2) * SL + sl;
     const int s = blockIdx.x;
     if (pair >= p.pairs) return;
     const int G = p.num_wg, X = p.switch_tiles;
     int T = 0, S = 0, K = 0, KS = 0;  // tiles and non-empty sequences: all, before s
-    for (int base = 0; base < p.num_seqs; base += 64) {
-        const int sl = base + lane;
-        const int nt = sl < p.num_seqs ? tiles_of(p, sl) : 0;
-        T += wave_sum(nt);
-        S += wave_sum(sl < s ? nt : 0);
-        K += wave_sum(nt > 0 ? 1 : 0);
-        KS += wave_sum(sl < s && nt > 0 ? 1 : 0);
+    for (int base = 0; base < p.num_seqs; base += 128) {
+        int nt[2];
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const int i = base + 64 * k + lane;
+            nt[k] = i < p.num_seqs ? tiles_of(p, i) : 0;
+        }
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const bool before = base + 64 * k + lane < s;
+            T += wave_sum(nt[k]);
+            S += wave_sum(before ? nt[k] : 0);
+            K += __builtin_popcountll(__ballot(nt[k] > 0));
+            KS += __builtin_popcountll(__ballot(before && nt[k] > 0));
+        }
     }
     const int E = S + tiles_of(p, s);
     if (E <= S) return;  // no tiles: zeroed by the decode kernel
@@ -726,9 +728,16 @@ __global__ __launch_bounds__(256) void merge_split_kernel(DecodeParams p) {
     const int w0 = sp.span_of(S + shift), w1 = sp.span_of(E - 1 + shift);
     if (w0 == w1) return;  // finished in place
     const int kvh = pair / p.qchunks, qc = pair - kvh * p.qchunks;
-    merge_fragments<D>(p, s, w0, w1, pair, kvh * p.group + qc * 8, min(8, p.group - qc * 8), sp,
-                       lane, reinterpret_cast<__attribute__((address_space(3))) float*>(
-                                 (__attribute__((address_space(3))) float*)wts_all[wave]));
+    const int n_out = min(8, p.group - qc * 8) * D;
+    const int e = 4 * (64 * unit + lane);
+    const bool act = e < n_out;
+    const int ec = act ? e : 0, h = ec / D;
+    const bool all = sp.sp.all_live();
+    float* out = p.out + ((int64_t)s * p.num_heads + kvh * p.group + qc * 8) * D + ec;
+    merge_unit<FW>(
+        w1 - w0 + 1, fw, lane, act, out, [&](int i) { return all || sp.live(w0 + i); },
+        [&](int i) { return p.ws_ml + frag_block(w0, i, p.pairs, pair) * 16 + h; },
+        [&](int i) { return p.ws_o + frag_block(w0, i, p.pairs, pair) * (8 * D) + ec; }, part + (FW > 1 ? sl * FW : 0));
 }
 
 // ---- fp32 pages -----------------------------------------------------------
@@ -886,49 +895,28 @@ __global__ __launch_bounds__(256) void decode_f32_kernel(DecodeParams p) {
     }
 }
 
-// Log-sum-exp merge of the fixed partitions of one (sequence, head) per wave.
-__global__ __launch_bounds__(256) void merge_parts_kernel(DecodeParams p) {
-    const int lane = threadIdx.x & 63;
-    const int head = blockIdx.y * 4 + (threadIdx.x >> 6);
+// Log-sum-exp merge of the fixed partitions: a workgroup of FW waves per
+// (sequence, 256 of its num_heads * head_dim outputs).
+template <int FW>
+__global__ __launch_bounds__(FW * 64) void merge_parts_kernel(DecodeParams p) {
+    __shared__ float part[FW][64][6];
+    const int lane = threadIdx.x & 63, fw = threadIdx.x >> 6;
     const int seq = blockIdx.x;
-    if (head >= p.num_heads) return;
     const int ctx = min(p.context_lens[seq], p.max_parts * p.partition);
     const int P = p.partition;
     const int np = ctx <= 0 ? 1 : min((ctx + P - 1) / P, p.max_parts);
     if (np <= 1) return;
     const int D = p.head_dim;
-    const int64_t base = (int64_t)seq * p.max_parts * p.num_heads + head;
-    float M = kMaxSeed, L = 0.f;
-    for (int i0 = 0; i0 < np; i0 += 64) {
-        const int i = i0 + lane;
-        float2 ml = make_float2(kMaxSeed, 0.f);
-        if (i < np) ml = p.ws_ml[base + (int64_t)i * p.num_heads];
-        float m = ml.x;
-        for (int k = 32; k >= 1; k >>= 1) m = fmaxf(m, shfl_xor(m, k));
-        const float Mn = fmaxf(M, m);
-        float l = fast_exp2(ml.x - Mn) * ml.y;
-        for (int k = 32; k >= 1; k >>= 1) l += shfl_xor(l, k);
-        L = L * fast_exp2(M - Mn) + l;
-        M = Mn;
-    }
-    const float inv = 1.0f / (L + 1e-9f);
-    float acc[4] = {0.f, 0.f, 0.f, 0.f};
-    for (int i0 = 0; i0 < np; i0 += 64) {
-        const int n = min(64, np - i0);
-        float wt = 0.f;
-        if (i0 + lane < np) wt = fast_exp2(p.ws_ml[base + (int64_t)(i0 + lane) * p.num_heads].x - M);
-        for (int j = 0; j < n; ++j) {
-            const float wj = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wt), j));
-            const float* orow = p.ws_o + (base + (int64_t)(i0 + j) * p.num_heads) * D;
-#pragma unroll
-            for (int k = 0; k < 4; ++k)
-                if (lane + 64 * k < D) acc[k] += wj * orow[lane + 64 * k];
-        }
-    }
-    float* out = p.out + ((int64_t)seq * p.num_heads + head) * D;
-#pragma unroll
-    for (int k = 0; k < 4; ++k)
-        if (lane + 64 * k < D) out[lane + 64 * k] = acc[k] * inv;
+    const int64_t n_out = (int64_t)p.num_heads * D;
+    const int64_t e = 4 * (64 * (blockIdx.y + (int64_t)gridDim.y * blockIdx.z) + lane);
+    const bool act = e < n_out;
+    const int64_t ec = act ? e : 0;
+    const int64_t base = (int64_t)seq * p.max_parts;
+    const float2* ml = p.ws_ml + base * p.num_heads + ec / D;
+    const float* o = p.ws_o + base * n_out + ec;
+    merge_unit<FW>(
+        np, fw, lane, act, p.out + (int64_t)seq * n_out + ec, [](int) { return true; },
+        [&](int i) { return ml + (int64_t)i * p.num_heads; }, [&](int i) { return o + (int64_t)i * n_out; }, part);
 }
 
 // ---------------------------------------------------------------------------
@@ -1722,6 +1710,53 @@ hipError_t launch_mfma(const DecodeParams& p, hipStream_t stream) {
     }
 }
 
+// Waves per merge unit (256 outputs of a sequence's row, `units` in all): the
+// merge's time is its rounds of loads for few units and its waves' fixed work
+// (each scans the context lengths) for many, so a unit gets 8 waves while
+// that keeps the launch at 2048 waves (two per SIMD), else 2, else 1.
+// Measured (us, 1 / 2 / 8 waves): one 32768-token sequence, 24 units of 256
+// fragments, 34.1 / 18.2 / 7.9; 16 x 32768, 384 units of 16, 5.2 / 4.7 / 5.1;
+// 40 sequences of 100..5000, 640 units of 13, 6.6 / 5.8 / 7.1; 64 of
+// 128..4096, 1536 units of 4, 4.8 / 4.9 / 9.4.
+int merge_waves(int64_t units) { return units * 8 <= 2048 ? 8 : units * 2 <= 2048 ? 2 : 1; }
+
+template <int D, int SL, int FW>
+hipError_t launch_merge_shape(const DecodeParams& p, int units, hipStream_t stream) {
+    const dim3 grid(p.num_seqs, (p.pairs + 3) / 4, (units + SL - 1) / SL * 4);
+    hipLaunchKernelGGL((merge_split_kernel<D, SL, FW>), grid, dim3(SL * FW * 64), 0, stream, p);
+    return hipGetLastError();
+}
+
+template <int D>
+hipError_t launch_merge_d(const DecodeParams& p, hipStream_t stream) {
+    const int units = (min(8, p.group) * D + 255) / 256;  // per (sequence, kv-head slot)
+    switch (merge_waves((int64_t)p.num_seqs * p.pairs * units)) {
+        case 8: return launch_merge_shape<D, 1, 8>(p, units, stream);
+        case 2: return launch_merge_shape<D, 1, 2>(p, units, stream);
+        default: return launch_merge_shape<D, (8 * D + 255) / 256, 1>(p, units, stream);
+    }
+}
+
+hipError_t launch_merge_split(const DecodeParams& p, hipStream_t stream) {
+    switch (p.head_dim) {
+        case 64: return launch_merge_d<64>(p, stream);
+        case 80: return launch_merge_d<80>(p, stream);
+        default: return launch_merge_d<128>(p, stream);
+    }
+}
+
+hipError_t launch_merge_parts(const DecodeParams& p, hipStream_t stream) {
+    const int64_t units = ((int64_t)p.num_heads * p.head_dim + 255) / 256;
+    const int64_t ny = std::min<int64_t>(units, 32768);
+    const dim3 grid(p.num_seqs, (unsigned)ny, (unsigned)((units + ny - 1) / ny));
+    switch (merge_waves(units * p.num_seqs)) {
+        case 8: hipLaunchKernelGGL(merge_parts_kernel<8>, grid, dim3(512), 0, stream, p); break;
+        case 2: hipLaunchKernelGGL(merge_parts_kernel<2>, grid, dim3(128), 0, stream, p); break;
+        default: hipLaunchKernelGGL(merge_parts_kernel<1>, grid, dim3(64), 0, stream, p); break;
+    }
+    return hipGetLastError();
+}
+
 }  // namespace
 
 int decode_group_count(int pairs) {
@@ -1757,9 +1792,7 @@ hipError_t launch_decode(const DecodeParams& p, hipStream_t stream, const MergeF
         if (prof) prof_end(kKernelDecode, stream);
         if (p.max_parts > 1) {
             if (prof) prof_begin(kKernelMerge, stream);
-            dim3 mg(p.num_seqs, (p.num_heads + 3) / 4);
-            hipLaunchKernelGGL(merge_parts_kernel, mg, dim3(256), 0, stream, p);
-            err = hipGetLastError();
+            err = launch_merge_parts(p, stream);
             if (prof) prof_end(kKernelMerge, stream);
         }
         return err;
@@ -1794,13 +1827,7 @@ hipError_t launch_decode(const DecodeParams& p, hipStream_t stream, const MergeF
         stream = mf->side;
     }
     if (prof) prof_begin(kKernelMerge, stream);
-    dim3 mg(p.num_seqs, (p.pairs + 3) / 4);
-    switch (p.head_dim) {
-        case 64: hipLaunchKernelGGL(merge_split_kernel<64>, mg, dim3(256), 0, stream, p); break;
-        case 80: hipLaunchKernelGGL(merge_split_kernel<80>, mg, dim3(256), 0, stream, p); break;
-        default: hipLaunchKernelGGL(merge_split_kernel<128>, mg, dim3(256), 0, stream, p); break;
-    }
-    err = hipGetLastError();
+    err = launch_merge_split(p, stream);
     if (prof) prof_end(kKernelMerge, stream);
     if (mf) {  // recorded even after a failed merge launch, so the caller can always join
         const hipError_t ej = hipEventRecord(mf->join, stream);
@@ -1875,10 +1902,7 @@ hipError_t launch_mixed(const DecodeParams& dp, const PrefillParams& pp, int cus
     if (err != hipSuccess) return err;
     if (prof) prof_end(kKernelMixed, stream);
     if (prof) prof_begin(kKernelMerge, stream);
-    dim3 mgr(dp.num_seqs, (dp.pairs + 3) / 4);
-    if (dp.head_dim == 64) hipLaunchKernelGGL(merge_split_kernel<64>, mgr, dim3(256), 0, stream, dp);
-    else hipLaunchKernelGGL(merge_split_kernel<80>, mgr, dim3(256), 0, stream, dp);
-    err = hipGetLastError();
+    err = launch_merge_split(dp, stream);
     if (prof) prof_end(kKernelMerge, stream);
     return err;
 }

@@ -16,7 +16,8 @@
 // group of 4 query heads); one wave per query head holds RB row blocks of 16
 // query tokens.  Keys stream in blocks of 32 through a ring of LDS stages that
 // the workgroup fills with direct-to-LDS DMA (global_load_lds_dwordx4, one
-// page lookup per lane, explicit vmcnt bookkeeping), two blocks per barrier.
+// page lookup per lane, explicit vmcnt bookkeeping), one or two blocks per
+// barrier (DmaDims::PER_BARRIER).
 // Byte pages (int8, FP8) arrive raw and are widened by the workgroup into an
 // fp16 area: FP8 to its values, int8 K to exact integers (its per-key scale
 // joins the exp's fma below) and int8 V to fp16(v * scale).  Per row block
@@ -106,6 +107,12 @@ struct DmaDims {
 #else
     static constexpr int STAGES = D <= 80 && !F ? 6 : 4; // ring depth (LDS: <= 64 KiB)
 #endif
+    // Key blocks consumed per barrier.  The deep rings take two; four stages
+    // (D = 128: two workgroups' rings fill the LDS) take one, since pairs
+    // would wait for the whole ring to drain before every pair: 8 chunks of
+    // 2048 tokens on 1024-token prefixes, 32 heads of 128, 638 -> 615 us, one
+    // 512-token chunk on 16384, 167 -> 162 us.
+    static constexpr int PER_BARRIER = STAGES >= 6 || F ? 2 : 1;
     static_assert((2 * REGION) % 64 == 0, "stage must be whole DMA instructions");
 };
 
@@ -553,14 +560,15 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int bx, int
         }
     };
 
-    // fp16 pages: a ring of kStages 32-key blocks, consumed two per barrier:
-    // while blocks kb, kb + 1 are computed, blocks up to kb + kStages - 1 are
-    // in flight.  Byte pages: a ring of kStages byte blocks and two fp16
+    // fp16 pages: a ring of kStages 32-key blocks, consumed PER_BARRIER (one
+    // or two) per barrier: while block kb (or kb, kb + 1) is computed, blocks
+    // up to kb + kStages - 1 are in flight.  Byte pages: a ring of kStages byte blocks and two fp16
     // blocks, one block per barrier: block kb is computed from its fp16 copy
     // while block kb + 1 is widened into the other one and blocks up to
     // kb + kStages - 2 are in flight.  Blocks past nblk are issued too (as
     // zero chunks) so that every wave's vmcnt arithmetic below stays exact;
-    // on fp16 pages an odd tail block is paired with a fully masked one.
+    // where fp16 pages take two, an odd tail block is paired with a fully
+    // masked one.
     static_assert(kStages >= 4 && kStages % 2 == 0, "ring holds whole pairs");
     const int free_end = any_bad ? 0 : (min(nfree, nblk) & ~1);
     if constexpr (BYTES) {
@@ -588,27 +596,29 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int bx, int
             compute(kb, std::true_type{});
         }
     } else {
+        // Blocks consumed per barrier.
+        constexpr int PB = DD::PER_BARRIER;
 #pragma unroll
-        for (int s = 0; s < kStages - 2; ++s) issue(kb_lo + s);
+        for (int s = 0; s < kStages - PB; ++s) issue(kb_lo + s);
         auto step = [&](int kb) {
-            constexpr int kAhead = kStages - 4;  // blocks allowed in flight at the wait
+            constexpr int kAhead = kStages - 2 * PB;  // blocks allowed in flight at the wait
             if (my_inst == PERW) wait_vmcnt<kAhead * PERW>();
             else wait_vmcnt<kAhead * (PERW - 1)>();
-            __syncthreads();  // blocks kb, kb + 1 landed for all waves; kb - 2, kb - 1 consumed
-            issue(kb + kStages - 2);
-            issue(kb + kStages - 1);
+            __syncthreads();  // blocks kb .. kb + PB - 1 landed for all waves; the PB before kb consumed
+#pragma unroll
+            for (int h = 0; h < PB; ++h) issue(kb + kStages - PB + h);
         };
         // Two loops, one inlined compute each (one loop with both variants
         // merges their accumulators and spills).
-        for (int kb = kb_lo; kb < min(free_end, kb_hi); kb += 2) {
+        for (int kb = kb_lo; kb < min(free_end, kb_hi); kb += PB) {
             step(kb);
 #pragma unroll 1
-            for (int h = 0; h < 2; ++h) compute(kb + h, std::false_type{});
+            for (int h = 0; h < PB; ++h) compute(kb + h, std::false_type{});
         }
-        for (int kb = max(free_end, kb_lo); kb < kb_hi; kb += 2) {
+        for (int kb = max(free_end, kb_lo); kb < kb_hi; kb += PB) {
             step(kb);
 #pragma unroll 1
-            for (int h = 0; h < 2; ++h) compute(kb + h, std::true_type{});
+            for (int h = 0; h < PB; ++h) compute(kb + h, std::true_type{});
         }
     }
     wait_vmcnt<0>();

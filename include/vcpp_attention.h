@@ -106,7 +106,9 @@ typedef struct vcpp_kv_pages {
  *                a larger context_len is an error the kernel cannot report:
  *                positions past max_context_len are not attended)
  *   partition_size   0 (default): the tiles of all sequences are split
- *                evenly over the workgroups the GPU holds at once (fp16/int8/fp8)
+ *                evenly over the workgroups the GPU holds at once (fp16/int8/fp8;
+ *                small batches: partitions of 64..1024 tokens, chosen so that
+ *                there are at most two workgroups per compute unit)
  *                or (fp32) into partitions of 32..256 tokens sized so the
  *                workgroups fill the GPU about twice.  > 0 (a multiple of 16,
  *                <= 1024): fixed partitions -- the tiles are split into

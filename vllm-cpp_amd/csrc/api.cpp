@@ -146,13 +146,34 @@ bool no_merge_fork() {
 // Launch geometry and workspace layout of one decode call.
 struct DecodePlan {
     int32_t num_wg = 0;      // fp16/int8: workgroup ranges per kv-head group
+    bool small = false;      // fp16/int8/fp8: small batch, decode_small_kernel
     bool page_mode = false;  // fp16/int8, Hkv 8: page-staged kernel
     int32_t page_grid = 0;   // page mode: workgroups (one per range, or a run of ranges each)
-    int32_t partition = 0;   // fp32: tokens per partition
-    int32_t max_parts = 0;   // fp32: partitions per sequence
+    int32_t partition = 0;   // fp32, small batches: tokens per partition
+    int32_t max_parts = 0;   // fp32, small batches: partitions per sequence
     int32_t g1 = 0, g1_share = 0;  // page mode: unequal ranges (see DecodeParams)
     size_t off_o = 0, off_ml = 0, bytes = 0;
 };
+
+// Partition of a small batch (0: not one): `units` (sequence, kv-head slot)
+// pairs of at most max_ctx tokens in fixed partitions, one workgroup each.
+// The smallest partition whose workgroups are at most two per CU, up to 512
+// tokens -- 1024 where the general path is the register kernel, which the
+// page-staged one beats.  Past that the general path's balanced split wins:
+// 4 x 16384 tokens (f16, 64/8 heads of 80) 43.6 us at 512 against 34.6, while
+// 1 x 32768 takes 23.7 against 26.6; register-path shapes (12/2 heads of 128)
+// 64 x 4096 at 1024, 51.0 against 61.0.  Up to 256 tokens one partition wins
+// outright (no merge: 4 x 256, 8.5 us against 9.4 at 64); up to 512 it does
+// where 64-token partitions would be too many (16 x 512, 14.0 against 14.5).
+int32_t small_partition(int64_t units, int32_t max_ctx, bool page_mode) {
+    const int64_t most = 2 * (int64_t)device_cus();
+    if (units > most || units > 65535) return 0;
+    if (max_ctx <= 256) return 256;
+    const int32_t top = page_mode ? 512 : 1024;
+    for (int32_t P = 64; P <= top; P *= 2)
+        if (units * num_parts(max_ctx, P) <= most) return max_ctx <= 512 && P > 64 ? 512 : P;
+    return 0;
+}
 
 // fused_grid > 0: the decode side of the fused mixed step, whose decode
 // workers (fused_grid per kv-head group of 4) walk the balanced split.
@@ -245,6 +266,21 @@ DecodePlan plan_decode(const vcpp_kv_pages* kv, int32_t num_seqs, int32_t num_he
     const size_t blocks = (size_t)G * 2 * pairs;  // [range][slot][kv-head slot]
     pl.off_ml = pl.off_o + align256(blocks * 8 * D * sizeof(float));
     pl.bytes = pl.off_ml + align256(blocks * 16 * sizeof(float2));
+    if (partition_size == 0 && fused_grid == 0 && !(pe && pe[0] == '0')) {
+        const int32_t P = small_partition((int64_t)num_seqs * pairs, max_context_len, pl.page_mode);
+        const int32_t parts = P > 0 ? num_parts(max_context_len, P) : 0;
+        const size_t rows = (size_t)num_seqs * parts * num_heads;
+        const size_t off_ml = align256(rows * D * sizeof(float));
+        // The workspace size stays the general plan's, which holds these
+        // partials (512 workgroups of at most 8 heads, fewer than its ranges'
+        // two blocks of 8); checked all the same.
+        if (parts == 1 || (parts > 1 && parts <= 65535 && off_ml + align256(rows * sizeof(float2)) <= pl.bytes)) {
+            pl.small = true;
+            pl.partition = P;
+            pl.max_parts = parts;
+            pl.off_ml = off_ml;
+        }
+    }
     return pl;
 }
 
@@ -470,6 +506,7 @@ vcpp::DecodeParams decode_params(const vcpp_kv_pages* kv, const float* q, float*
     p.partition = pl.partition;
     p.max_parts = pl.max_parts;
     p.num_wg = pl.num_wg;
+    p.small = pl.small ? 1 : 0;
     p.page_mode = pl.page_mode ? 1 : 0;
     p.page_grid = pl.page_grid;
     p.g1 = pl.g1;

@@ -44,15 +44,17 @@ struct DecodeParams {
     // preceded by switch_tiles units that hold no tile (0: plain tile split).
     int32_t switch_tiles;
     int32_t ctx_cap;       // context lengths are clamped to this
-    // fp32: fixed partitions of `partition` tokens, max_parts per sequence
+    // fp32, and small batches: fixed partitions of `partition` tokens, max_parts
+    // per sequence
     int32_t partition;
     int32_t max_parts;
     // partials: fp16/int8 blocks [num_wg][2 slots][pairs] of [8 heads][head_dim] outputs and
-    // 16 (m, l) pairs; fp32 [num_seqs][max_parts][num_heads]
+    // 16 (m, l) pairs; fp32 and small batches [num_seqs][max_parts][num_heads]
     float* ws_o;     // (.., head_dim) unnormalised outputs
     float2* ws_ml;   // (max in log2 units, sum of exponentials)
     float scale_log2;  // log2(e) / sqrt(head_dim)
     int32_t pipeline;  // fp16/int8 pipeline shape (tuning; 0 = default)
+    int32_t small;     // fp16/int8/fp8: decode_small_kernel over fixed partitions
     int32_t page_mode; // fp16/int8, Hkv 8: 8-wave workgroups staging whole tiles in LDS
     int32_t page_grid; // workgroups that walk the num_wg ranges (page mode: a run each; else num_wg)
     // Balanced page split (one range per workgroup), g1 > 0: ranges of

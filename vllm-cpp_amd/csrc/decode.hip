@@ -6,7 +6,9 @@
 // The reference's GPU slot is cuda/attention.cu:11-52; its kernel
 // (cuda/attention_kernels.cuh:9-123) is not followed.
 //
-// fp16 / int8 / FP8 pages (the HBM-bound path) run one of two kernels with the
+// fp16 / int8 / FP8 pages run one of three kernels.  Small batches take
+// decode_small_kernel (fixed partitions, at most two workgroups per CU in
+// all; its own comment).  The HBM-bound rest runs one of two kernels with the
 // same split, MFMA step and merge (below).
 //  * decode_page_kernel -- Hkv = 8, <= 8 query heads per kv head, D 64 or 80:
 //    a workgroup of 8 waves (one per kv head) walks its range of 16-token
@@ -387,8 +389,8 @@ __device__ __forceinline__ void merge_unit(int nfr, int fw, int lane, bool act, 
 #pragma unroll
         for (int j = 0; j < kMergeChunk; ++j) {
             const float w = live[j] ? fast_exp2(x[j].x - Mn) : 0.f;
-            L += w * x[j].y;
-            acc += w * v[j];
+            L += live[j] ? w * x[j].y : 0.f;
+            acc += live[j] ? w * v[j] : f4{0.f, 0.f, 0.f, 0.f};
         }
     }
     if constexpr (FW > 1) {
@@ -417,10 +419,214 @@ __device__ __forceinline__ void merge_unit(int nfr, int fw, int lane, bool act, 
     if (act) *reinterpret_cast<f4*>(out) = acc * (1.0f / (L + 1e-9f));
 }
 
+// One wave's attention of 8 query heads of a kv head over a list of 16-token
+// tiles of one sequence, K and V loaded straight from the pages into
+// registers.  The state is the online softmax (m_run, l_run per head column)
+// and the output accumulators of the hi / lo rows.
+template <int KV, int D, int TPS, int NBUF, bool MASK_ALL = false>
+struct WaveAttn {
+    static constexpr int NC32 = Dims<D>::NC32, NT = Dims<D>::NT;
+    h8 qa[NC32 > 0 ? NC32 : 1];
+    h4 qr;
+    f4 o[NT];
+    float m_run, l_run;
+
+    // Query fragment: row c = hi (c < 8) or lo (c >= 8) of head c & 7.
+    __device__ __forceinline__ void load_q(const DecodeParams& p, int s, int head_base, int gc, int g, int c) {
+        const bool qv = (c & 7) < gc;
+        const float* qrow = p.q + ((int64_t)s * p.num_heads + head_base + (c & 7)) * D;
+        qr = h4{};
+#pragma unroll
+        for (int cc = 0; cc < NC32; ++cc) {
+            f4 x0 = {}, x1 = {};
+            if (qv) {
+                x0 = *reinterpret_cast<const f4*>(qrow + 32 * cc + 8 * g);
+                x1 = *reinterpret_cast<const f4*>(qrow + 32 * cc + 8 * g + 4);
+            }
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const float x = i < 4 ? x0[i] : x1[i - 4];
+                const _Float16 hi = (_Float16)x;
+                qa[cc][i] = c < 8 ? hi : (_Float16)(x - (float)hi);
+            }
+        }
+        if constexpr (Dims<D>::REM) {
+            f4 x = {};
+            if (qv) x = *reinterpret_cast<const f4*>(qrow + 32 * NC32 + 4 * g);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const _Float16 hi = (_Float16)x[i];
+                qr[i] = c < 8 ? hi : (_Float16)(x[i] - (float)hi);
+            }
+        }
+    }
+
+    __device__ __forceinline__ void start() {
+#pragma unroll
+        for (int t = 0; t < NT; ++t) o[t] = f4{0.f, 0.f, 0.f, 0.f};
+        m_run = kMaxSeed;
+        l_run = 0.f;
+    }
+
+    // Tiles first, first + stride, .. (ntiles <= 64 of them); lane j holds the
+    // physical block (-1: zeros) and the first token in it of the j-th.
+    // Positions at or past `end` are masked.  lds: the wave's TPS V tiles.
+    __device__ __forceinline__ void run(const DecodeParams& p, int s, int pair, int my_bid, int my_off, int ntiles,
+                                        int first, int stride, int end, const LaneOffsets& lofs, lds_char* lds,
+                                        int lane) {
+        const int g = lane >> 4, c = lane & 15;
+        auto load_step = [&](Tile<KV, D>(&buf)[TPS], int it) {
+#pragma unroll
+            for (int j = 0; j < TPS; ++j) {
+                const int tt = it * TPS + j;
+                const int bid = tt < ntiles ? __builtin_amdgcn_readlane(my_bid, tt & 63) : -1;
+                const int off = __builtin_amdgcn_readlane(my_off, tt & 63);
+#ifdef VCPP_GATHER_DUMP
+                const int gpos = (first + stride * tt) * kTile + lane;
+                if (pair == 0 && tt < ntiles && lane < kTile && bid >= 0 && gpos < end)
+                    gather_record(p, s, gpos, bid, off + lane);
+#endif
+                load_tile<KV, D>(buf[j], p, bid, off, lofs);
+            }
+        };
+
+        // FULL: every tile of the step is a valid block lying wholly below `end`,
+        // so no masking code runs (the common case).
+        auto compute_step = [&](const Tile<KV, D>(&cur)[TPS], int it, auto full_tag) {
+            constexpr bool FULL = decltype(full_tag)::value;
+            float sc[TPS][4];
+            float mx = kMaxSeed;
+#pragma unroll
+            for (int j = 0; j < TPS; ++j) {
+                const int tt = it * TPS + j;
+                const int bid = tt < ntiles ? __builtin_amdgcn_readlane(my_bid, tt & 63) : -1;
+                const int pos0 = (first + stride * tt) * kTile;
+                const bool full = FULL || (bid >= 0 && pos0 + kTile <= end);  // wave-uniform
+                f4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int cc = 0; cc < NC32; ++cc)
+                    acc = mfma32(k_chunk<KV, D>(cur[j], cc), qa[cc], acc);
+                if constexpr (Dims<D>::REM) {
+                    // Own accumulator, summed on the VALU (see Dims).
+                    const f4 zero = {0.f, 0.f, 0.f, 0.f};
+                    const f4 acc2 = mfma16(k_rem<KV, D>(cur[j]), qr, zero);
+                    acc += acc2;
+                }
+                stage_v<KV, D>(lds + j * kTile * D * 2, cur[j], full || pos0 + c < end, g, c);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    float x = acc[r] + dpp_ror8(acc[r]);
+                    float f = p.scale_log2;
+                    if constexpr (KV == VCPP_KV_I8) {
+                        const uint32_t wd = (uint32_t)(r < 2 ? cur[j].ks.x : cur[j].ks.y);
+                        f *= h_to_f((r & 1) ? (wd >> 16) : (wd & 0xFFFFu));
+                    }
+                    x *= f;
+                    if (!full) x = (bid >= 0 && pos0 + 4 * g + r < end) ? x : -__builtin_inff();
+                    sc[j][r] = x;
+                    mx = fmaxf(mx, x);
+                }
+            }
+            mx = fmaxf(mx, shfl_xor(mx, 16));
+            mx = fmaxf(mx, shfl_xor(mx, 32));
+            const float m_new = fmaxf(m_run, mx);
+            const float alpha = fast_exp2(m_run - m_new);
+            m_run = m_new;
+            if (__any(alpha != 1.0f)) {
+                // Accumulator row 4g + r belongs to head (4g + r) & 7.
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float al = shfl(alpha, (4 * g + r) & 7);
+#pragma unroll
+                    for (int t = 0; t < NT; ++t) o[t][r] *= al;
+                }
+            }
+            float lsum = 0.f;
+#pragma unroll
+            for (int j = 0; j < TPS; ++j) {
+                h4 pa;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    float pr = fast_exp2(sc[j][r] - m_new);
+                    lsum += pr;
+                    if constexpr (KV == VCPP_KV_I8) {
+                        const uint32_t wd = (uint32_t)(r < 2 ? cur[j].vs.x : cur[j].vs.y);
+                        // masked tokens have pr == 0; the select keeps 0 * garbage out
+                        pr = pr > 0.f ? pr * h_to_f((r & 1) ? (wd >> 16) : (wd & 0xFFFFu)) : 0.f;
+                    }
+                    const _Float16 hi = (_Float16)pr;
+                    pa[r] = c < 8 ? hi : (_Float16)(pr - (float)hi);
+                }
+                lds_char* vt = lds + j * kTile * D * 2;
+#pragma unroll
+                for (int t = 0; t < NT; ++t) o[t] = mfma16(pa, read_v_tr<D>(vt, t, g, c), o[t]);
+            }
+            l_run = l_run * alpha + lsum;
+        };
+
+        // NBUF register buffers in rotation: steps it+1 .. it+NBUF-1 are in
+        // flight while step it computes; no buffer is copied (a copy would
+        // wait on its loads).  Steps past the end load zero-sized (free) tiles.
+        Tile<KV, D> buf[NBUF][TPS];
+        const int niters = (ntiles + TPS - 1) / TPS;
+        // Whole steps of valid blocks below `end` (tiles are in order).
+        int nfull = 0;
+        {
+            const int last_ok = ((first + stride * (ntiles - 1) + 1) * kTile <= end);
+            const bool all_valid = __builtin_amdgcn_read_exec() ==
+                                   (uint64_t)__ballot(lane >= ntiles || my_bid >= 0);
+            const int full_tiles = all_valid ? (last_ok ? ntiles : ntiles - 1) : 0;
+            nfull = full_tiles / TPS;
+        }
+#pragma unroll
+        for (int k = 0; k < NBUF - 1; ++k) load_step(buf[k], k);
+        for (int it = 0; it < niters; it += NBUF) {
+#pragma unroll
+            for (int k = 0; k < NBUF; ++k) {
+                if (it + k >= niters) break;
+                load_step(buf[(k + NBUF - 1) % NBUF], it + k + NBUF - 1);
+                if (!MASK_ALL && it + k < nfull) compute_step(buf[k], it + k, std::true_type{});
+                else compute_step(buf[k], it + k, std::false_type{});
+            }
+        }
+    }
+
+    // Per-head totals of this wave: O rows h (hi) + h + 8 (lo) summed in
+    // place (lane (g, c), g < 2: heads 4 g + r, columns 16 t + c), and the
+    // heads' (max, sum) of those rows.
+    __device__ __forceinline__ void finish(int g, float (&mh)[4], float (&lh)[4]) {
+        float lt = l_run;
+        lt += shfl_xor(lt, 16);
+        lt += shfl_xor(lt, 32);
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) o[t][r] += shfl_xor(o[t][r], 32);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            lh[r] = shfl(lt, (4 * g + r) & 7);
+            mh[r] = shfl(m_run, (4 * g + r) & 7);
+        }
+    }
+};
+
+// Physical block of tile `t` of sequence s (-1: past the table or an id
+// outside the pool) and its first token there.
+__device__ __forceinline__ void lookup_tile(const DecodeParams& p, int s, int t, int tlen, int& bid, int& off) {
+    const int pos = t * kTile;
+    const int lb = pos / p.block_size;
+    off = pos - lb * p.block_size;
+    bid = -1;
+    if (lb < tlen) {
+        const int id = p.block_tables[(int64_t)s * p.max_blocks + lb];
+        if (id >= 0 && (int64_t)id < p.num_blocks) bid = id;
+    }
+}
+
 template <int KV, int D, int TPS, int NBUF>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void decode_mfma_kernel(DecodeParams p) {
-    constexpr int NC32 = Dims<D>::NC32, NT = Dims<D>::NT;
+    constexpr int NT = Dims<D>::NT;
     extern __shared__ char lds_raw[];
 
     const int lane = threadIdx.x & 63;
@@ -457,187 +663,19 @@ void decode_mfma_kernel(DecodeParams p) {
         if (p.table_lens) tlen = min(tlen, p.table_lens[s]);
         const int end = (int)min((int64_t)ctx, (int64_t)tlen * p.block_size);
 
-        // Query fragment: row c = hi (c < 8) or lo (c >= 8) of head c & 7.
-        h8 qa[NC32 > 0 ? NC32 : 1];
-        h4 qr = {};
-        {
-            const bool qv = (c & 7) < gc;
-            const float* qrow = p.q + ((int64_t)s * p.num_heads + head_base + (c & 7)) * D;
-#pragma unroll
-            for (int cc = 0; cc < NC32; ++cc) {
-                f4 x0 = {}, x1 = {};
-                if (qv) {
-                    x0 = *reinterpret_cast<const f4*>(qrow + 32 * cc + 8 * g);
-                    x1 = *reinterpret_cast<const f4*>(qrow + 32 * cc + 8 * g + 4);
-                }
-#pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    const float x = i < 4 ? x0[i] : x1[i - 4];
-                    const _Float16 hi = (_Float16)x;
-                    qa[cc][i] = c < 8 ? hi : (_Float16)(x - (float)hi);
-                }
-            }
-            if constexpr (Dims<D>::REM) {
-                f4 x = {};
-                if (qv) x = *reinterpret_cast<const f4*>(qrow + 32 * NC32 + 4 * g);
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const _Float16 hi = (_Float16)x[i];
-                    qr[i] = c < 8 ? hi : (_Float16)(x[i] - (float)hi);
-                }
-            }
-        }
-
-        f4 o[NT];
-#pragma unroll
-        for (int t = 0; t < NT; ++t) o[t] = f4{0.f, 0.f, 0.f, 0.f};
-        float m_run = kMaxSeed, l_run = 0.f;
-
+        WaveAttn<KV, D, TPS, NBUF> wa;
+        wa.load_q(p, s, head_base, gc, g, c);
+        wa.start();
         for (int ch = t0; ch < t1; ch += 64) {
             const int ntiles = min(64, t1 - ch);
-            // Physical block of tile ch + j in lane j (-1: past the table or
-            // an id outside the pool).
+            // Physical block of tile ch + j in lane j.
             int my_bid = -1, my_off = 0;
-            if (lane < ntiles) {
-                const int pos = (ch + lane) * kTile;
-                const int lb = pos / p.block_size;
-                my_off = pos - lb * p.block_size;
-                if (lb < tlen) {
-                    const int id = p.block_tables[(int64_t)s * p.max_blocks + lb];
-                    if (id >= 0 && (int64_t)id < p.num_blocks) my_bid = id;
-                }
-            }
-
-            auto load_step = [&](Tile<KV, D>(&buf)[TPS], int it) {
-#pragma unroll
-                for (int j = 0; j < TPS; ++j) {
-                    const int tt = it * TPS + j;
-                    const int bid = tt < ntiles ? __builtin_amdgcn_readlane(my_bid, tt & 63) : -1;
-                    const int off = __builtin_amdgcn_readlane(my_off, tt & 63);
-#ifdef VCPP_GATHER_DUMP
-                    const int gpos = (ch + tt) * kTile + lane;
-                    if (pair == 0 && tt < ntiles && lane < kTile && bid >= 0 && gpos < end)
-                        gather_record(p, s, gpos, bid, off + lane);
-#endif
-                    load_tile<KV, D>(buf[j], p, bid, off, lofs);
-                }
-            };
-
-            // FULL: every tile of the step is a valid block lying wholly below `end`,
-            // so no masking code runs (the common case).
-            auto compute_step = [&](const Tile<KV, D>(&cur)[TPS], int it, auto full_tag) {
-                constexpr bool FULL = decltype(full_tag)::value;
-                float sc[TPS][4];
-                float mx = kMaxSeed;
-#pragma unroll
-                for (int j = 0; j < TPS; ++j) {
-                    const int tt = it * TPS + j;
-                    const int bid = tt < ntiles ? __builtin_amdgcn_readlane(my_bid, tt & 63) : -1;
-                    const int pos0 = (ch + tt) * kTile;
-                    const bool full = FULL || (bid >= 0 && pos0 + kTile <= end);  // wave-uniform
-                    f4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                    for (int cc = 0; cc < NC32; ++cc)
-                        acc = mfma32(k_chunk<KV, D>(cur[j], cc), qa[cc], acc);
-                    if constexpr (Dims<D>::REM) {
-                        // Own accumulator, summed on the VALU (see Dims).
-                        const f4 zero = {0.f, 0.f, 0.f, 0.f};
-                        const f4 acc2 = mfma16(k_rem<KV, D>(cur[j]), qr, zero);
-                        acc += acc2;
-                    }
-                    stage_v<KV, D>(lds + j * kTile * D * 2, cur[j], full || pos0 + c < end, g, c);
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        float x = acc[r] + dpp_ror8(acc[r]);
-                        float f = p.scale_log2;
-                        if constexpr (KV == VCPP_KV_I8) {
-                            const uint32_t wd = (uint32_t)(r < 2 ? cur[j].ks.x : cur[j].ks.y);
-                            f *= h_to_f((r & 1) ? (wd >> 16) : (wd & 0xFFFFu));
-                        }
-                        x *= f;
-                        if (!full) x = (bid >= 0 && pos0 + 4 * g + r < end) ? x : -__builtin_inff();
-                        sc[j][r] = x;
-                        mx = fmaxf(mx, x);
-                    }
-                }
-                mx = fmaxf(mx, shfl_xor(mx, 16));
-                mx = fmaxf(mx, shfl_xor(mx, 32));
-                const float m_new = fmaxf(m_run, mx);
-                const float alpha = fast_exp2(m_run - m_new);
-                m_run = m_new;
-                if (__any(alpha != 1.0f)) {
-                    // Accumulator row 4g + r belongs to head (4g + r) & 7.
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const float al = shfl(alpha, (4 * g + r) & 7);
-#pragma unroll
-                        for (int t = 0; t < NT; ++t) o[t][r] *= al;
-                    }
-                }
-                float lsum = 0.f;
-#pragma unroll
-                for (int j = 0; j < TPS; ++j) {
-                    h4 pa;
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        float pr = fast_exp2(sc[j][r] - m_new);
-                        lsum += pr;
-                        if constexpr (KV == VCPP_KV_I8) {
-                            const uint32_t wd = (uint32_t)(r < 2 ? cur[j].vs.x : cur[j].vs.y);
-                            // masked tokens have pr == 0; the select keeps 0 * garbage out
-                            pr = pr > 0.f ? pr * h_to_f((r & 1) ? (wd >> 16) : (wd & 0xFFFFu)) : 0.f;
-                        }
-                        const _Float16 hi = (_Float16)pr;
-                        pa[r] = c < 8 ? hi : (_Float16)(pr - (float)hi);
-                    }
-                    lds_char* vt = lds + j * kTile * D * 2;
-#pragma unroll
-                    for (int t = 0; t < NT; ++t) o[t] = mfma16(pa, read_v_tr<D>(vt, t, g, c), o[t]);
-                }
-                l_run = l_run * alpha + lsum;
-            };
-
-            // NBUF register buffers in rotation: steps it+1 .. it+NBUF-1 are in
-            // flight while step it computes; no buffer is copied (a copy would
-            // wait on its loads).  Steps past the end load zero-sized (free) tiles.
-            Tile<KV, D> buf[NBUF][TPS];
-            const int niters = (ntiles + TPS - 1) / TPS;
-            // Whole steps of valid blocks below `end` (tiles are in order).
-            int nfull = 0;
-            {
-                const int last_ok = (ch * kTile + ntiles * kTile <= end);
-                const bool all_valid = __builtin_amdgcn_read_exec() ==
-                                       (uint64_t)__ballot(lane >= ntiles || my_bid >= 0);
-                const int full_tiles = all_valid ? (last_ok ? ntiles : ntiles - 1) : 0;
-                nfull = full_tiles / TPS;
-            }
-#pragma unroll
-            for (int k = 0; k < NBUF - 1; ++k) load_step(buf[k], k);
-            for (int it = 0; it < niters; it += NBUF) {
-#pragma unroll
-                for (int k = 0; k < NBUF; ++k) {
-                    if (it + k >= niters) break;
-                    load_step(buf[(k + NBUF - 1) % NBUF], it + k + NBUF - 1);
-                    if (it + k < nfull) compute_step(buf[k], it + k, std::true_type{});
-                    else compute_step(buf[k], it + k, std::false_type{});
-                }
-            }
+            if (lane < ntiles) lookup_tile(p, s, ch + lane, tlen, my_bid, my_off);
+            wa.run(p, s, pair, my_bid, my_off, ntiles, ch, 1, end, lofs, lds, lane);
         }
 
-        // Per-head totals: l over the four lane groups; O rows h (hi) + h + 8 (lo).
-        float lt = l_run;
-        lt += shfl_xor(lt, 16);
-        lt += shfl_xor(lt, 32);
-#pragma unroll
-        for (int t = 0; t < NT; ++t)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) o[t][r] += shfl_xor(o[t][r], 32);
         float lh[4], mh[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            lh[r] = shfl(lt, (4 * g + r) & 7);
-            mh[r] = shfl(m_run, (4 * g + r) & 7);
-        }
+        wa.finish(g, mh, lh);
         if (g < 2) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
@@ -648,12 +686,12 @@ void decode_mfma_kernel(DecodeParams p) {
                     const float inv = 1.0f / (lh[r] + 1e-9f);
                     float* orow = p.out + ((int64_t)s * p.num_heads + head) * D;
 #pragma unroll
-                    for (int t = 0; t < NT; ++t) orow[16 * t + c] = o[t][r] * inv;
+                    for (int t = 0; t < NT; ++t) orow[16 * t + c] = wa.o[t][r] * inv;
                 } else {
                     const int64_t blk = ((int64_t)w * 2 + slot) * p.pairs + pair;
                     float* orow = p.ws_o + (blk * 8 + h) * D;
 #pragma unroll
-                    for (int t = 0; t < NT; ++t) orow[16 * t + c] = o[t][r];
+                    for (int t = 0; t < NT; ++t) orow[16 * t + c] = wa.o[t][r];
                     if (c == 0) p.ws_ml[blk * 16 + h] = make_float2(mh[r], lh[r]);
                 }
             }
@@ -687,6 +725,104 @@ void decode_mfma_kernel(DecodeParams p) {
             process_fragment(s, S, E);
         }
         if (carry >= b && !zero_owner_tail) break;
+    }
+}
+
+// ---- small batches ----------------------------------------------------------
+//
+// A workgroup of kSmallWaves waves per (sequence, kv-head slot, partition of
+// p.partition tokens): wave w takes the partition's tiles w, w + 4, ..
+// (register path, WaveAttn) and the waves' partials meet in LDS.  A sequence
+// of one partition is finished in place; longer ones leave partials for
+// merge_parts_kernel.
+//
+// The chain of round trips bounds a call this small, and the tile list, split
+// scan and DMA ring of the page-staged kernel make it longer: here the context
+// length, the block-table entries (a tile's place does not depend on the
+// length) and q are one round of loads, and the K/V tiles the next.
+// Code size counts as a round trip too (a launch this short runs its code
+// once, from a cold instruction cache): one tile per step, one buffer and one
+// masked form of it took 6.8 us for 128 tokens of 4 sequences (32/8 heads of
+// 128, fp16 pages) against 8.9 for the register kernel's four buffers and two
+// forms.  Four waves per SIMD hide the loads instead.
+// Kernel plus merge against the page-staged kernel and its merge (us, fp16,
+// 32/8 heads of 128, uniform contexts of half the maximum and up): 4 x 128
+// 6.6 against 17.7, 4 x 1024 11.7 against 17.8, 16 x 1024 18.7 against 23.7,
+// 16 x 2048 28.4 against 33.4; the rule is plan_decode's.
+constexpr int kSmallWaves = 4;
+
+template <int KV, int D>
+__global__ __launch_bounds__(kSmallWaves * 64) __attribute__((amdgpu_waves_per_eu(4, 4)))
+void decode_small_kernel(DecodeParams p) {
+    constexpr int NT = Dims<D>::NT, W = kSmallWaves;
+    constexpr int PO = 8 * D;  // a wave's partial outputs (floats), or its V tile (as many bytes)
+    __shared__ __attribute__((aligned(16))) char smem[W * PO * 4];
+    __shared__ float2 ml_s[W][8];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int g = lane >> 4, c = lane & 15;
+    const int s = blockIdx.x, pair = blockIdx.y, part = blockIdx.z;
+    const int kvh = pair / p.qchunks, qc = pair - kvh * p.qchunks;
+    const int head_base = kvh * p.group + qc * 8;
+    const int gc = min(8, p.group - qc * 8);
+    lds_char* lds = reinterpret_cast<lds_char*>((__attribute__((address_space(3))) char*)smem) + wave * PO * 4;
+
+    // One round of loads: the lengths, the first 64 tiles' block ids, q.
+    const int ctx = min(max(p.context_lens[s], 0), p.ctx_cap);
+    int tlen = p.max_blocks;
+    if (p.table_lens) tlen = min(tlen, p.table_lens[s]);
+    const int pt = p.partition / kTile;            // tiles per partition
+    const int first = part * pt + wave;
+    int my_bid, my_off;
+    lookup_tile(p, s, first + W * lane, p.max_blocks, my_bid, my_off);
+    WaveAttn<KV, D, 1, 1, true> wa;
+    wa.load_q(p, s, head_base, gc, g, c);
+    wa.start();
+    const LaneOffsets lofs = lane_offsets<KV, D>(p, kvh, g, c);
+
+    const int np = max(1, (ctx + p.partition - 1) / p.partition);  // partitions of the sequence
+    if (part >= np) return;                                        // whole workgroup
+    const int n = min((ctx + kTile - 1) / kTile, (part + 1) * pt);  // end of the partition's tiles
+    const int end = (int)min((int64_t)ctx, (int64_t)tlen * p.block_size);
+    for (int t0 = first; t0 < n; t0 += W * 64) {
+        const int ntiles = min(64, (n - t0 + W - 1) / W);
+        if (t0 != first) lookup_tile(p, s, t0 + W * lane, p.max_blocks, my_bid, my_off);
+        const bool in = lane < ntiles && (int64_t)(t0 + W * lane) * kTile < (int64_t)tlen * p.block_size;
+        wa.run(p, s, pair, in ? my_bid : -1, my_off, ntiles, t0, W, end, lofs, lds, lane);
+    }
+    float mh[4], lh[4];
+    wa.finish(g, mh, lh);
+    __syncthreads();  // the V tiles are read: their LDS takes the partials
+    float* po = reinterpret_cast<float*>(smem);
+    if (g < 2) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int h = 4 * g + r;
+#pragma unroll
+            for (int t = 0; t < NT; ++t) po[(wave * 8 + h) * D + 16 * t + c] = wa.o[t][r];
+            if (c == 0) ml_s[wave][h] = make_float2(mh[r], lh[r]);
+        }
+    }
+    __syncthreads();
+    const int e = 4 * threadIdx.x;  // 8 D <= 4 * threads
+    if (e >= gc * D) return;
+    const int h = e / D;
+    float M = kMaxSeed;
+#pragma unroll
+    for (int w = 0; w < W; ++w) M = fmaxf(M, ml_s[w][h].x);
+    float L = 0.f;
+    f4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+        const float wt = fast_exp2(ml_s[w][h].x - M);  // a wave without tiles: l = 0, o = 0
+        L += wt * ml_s[w][h].y;
+        acc += wt * *reinterpret_cast<const f4*>(po + w * PO + e);
+    }
+    if (np == 1) {
+        *reinterpret_cast<f4*>(p.out + ((int64_t)s * p.num_heads + head_base) * D + e) = acc * (1.0f / (L + 1e-9f));
+    } else {
+        const int64_t row = ((int64_t)s * p.max_parts + part) * p.num_heads + head_base;
+        *reinterpret_cast<f4*>(p.ws_o + row * D + e) = acc;
+        if (e - h * D == 0) p.ws_ml[row + h] = make_float2(M, L);
     }
 }
 
@@ -1757,6 +1893,18 @@ hipError_t launch_merge_parts(const DecodeParams& p, hipStream_t stream) {
     return hipGetLastError();
 }
 
+template <int KV>
+hipError_t launch_small(const DecodeParams& p, hipStream_t stream) {
+    const dim3 grid(p.num_seqs, p.pairs, p.max_parts), block(kSmallWaves * 64);
+    switch (p.head_dim) {
+        case 64: hipLaunchKernelGGL((decode_small_kernel<KV, 64>), grid, block, 0, stream, p); break;
+        case 80: hipLaunchKernelGGL((decode_small_kernel<KV, 80>), grid, block, 0, stream, p); break;
+        case 128: hipLaunchKernelGGL((decode_small_kernel<KV, 128>), grid, block, 0, stream, p); break;
+        default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+
 }  // namespace
 
 int decode_group_count(int pairs) {
@@ -1805,7 +1953,11 @@ hipError_t launch_decode(const DecodeParams& p, hipStream_t stream, const MergeF
         case 128: err = launch_mfma<KVT, 128>(p, stream); break;          \
         default: return hipErrorInvalidValue;                             \
     }
-    if (p.page_mode) {
+    if (p.small) {
+        if (p.kv_dtype == VCPP_KV_I8) err = launch_small<VCPP_KV_I8>(p, stream);
+        else if (p.kv_dtype == VCPP_KV_FP8) err = launch_small<VCPP_KV_FP8>(p, stream);
+        else err = launch_small<VCPP_KV_F16>(p, stream);
+    } else if (p.page_mode) {
         if (p.kv_dtype == VCPP_KV_I8) err = launch_page_kv<VCPP_KV_I8>(p, stream);
         else if (p.kv_dtype == VCPP_KV_FP8) err = launch_page_kv<VCPP_KV_FP8>(p, stream);
         else err = launch_page_kv<VCPP_KV_F16>(p, stream);
@@ -1819,6 +1971,7 @@ hipError_t launch_decode(const DecodeParams& p, hipStream_t stream, const MergeF
 #undef VCPP_DISPATCH_D
     if (err != hipSuccess) return err;
     if (prof) prof_end(kKernelDecode, stream);
+    if (p.small && p.max_parts == 1) return hipSuccess;  // finished in place
     if (mf) {
         err = hipEventRecord(mf->fork, stream);
         if (err == hipSuccess) err = hipStreamWaitEvent(mf->side, mf->fork, 0);
@@ -1827,7 +1980,7 @@ hipError_t launch_decode(const DecodeParams& p, hipStream_t stream, const MergeF
         stream = mf->side;
     }
     if (prof) prof_begin(kKernelMerge, stream);
-    err = launch_merge_split(p, stream);
+    err = p.small ? launch_merge_parts(p, stream) : launch_merge_split(p, stream);
     if (prof) prof_end(kKernelMerge, stream);
     if (mf) {  // recorded even after a failed merge launch, so the caller can always join
         const hipError_t ej = hipEventRecord(mf->join, stream);

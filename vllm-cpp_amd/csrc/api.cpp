@@ -939,7 +939,7 @@ void flash_attention_cuda(const float* q, const float* k, const float* v, float*
         fail(VCPP_E_UNSUPPORTED, "flash_attention_cuda: shape too large");
         return;
     }
-    vcpp::DenseParams p{q, k, v, out, attn_weights, attn_mask, batch_size, num_heads, head_dim, q_len, kv_len};
+    vcpp::DenseParams p{q, k, v, out, attn_weights, attn_mask, batch_size, num_heads, head_dim, q_len, kv_len, 1, kv_len};
     const hipError_t e = vcpp::launch_dense(p, nullptr);
     if (e != hipSuccess) hip_fail(e, "flash_attention_cuda launch");
 }

@@ -14,6 +14,8 @@ struct DenseParams {
     float* attn_weights; // [batch * heads][kv_len]
     const float* mask;   // [kv_len] or nullptr
     int32_t batch, heads, head_dim, q_len, kv_len;
+    // set by launch_dense where a pair's keys are split over workgroups
+    int32_t parts, part_keys;
 };
 
 hipError_t launch_dense(const DenseParams& p, hipStream_t stream);

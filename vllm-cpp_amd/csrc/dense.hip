@@ -7,10 +7,13 @@
 // same on the device: logits (and the mask, attn_mask[s] < 0 -> -1e9) into
 // attn_weights, a workgroup max and sum, probabilities back into
 // attn_weights, then out[d] = sum_s w[s] v[s][d] with one thread per d.
-// fp32 throughout; this is not a hot path.
+// fp32 throughout.  The shapes of dense_attention_dma_kernel (below) make one
+// pass over K and V, and few pairs split their keys over the idle CUs.
 #include "dense.h"
 
+#include <algorithm>
 #include <cstdlib>
+#include <mutex>
 
 #ifndef VCPP_DENSE_NW
 #define VCPP_DENSE_NW 4
@@ -226,18 +229,31 @@ __device__ __forceinline__ void dense_wait_vm() {
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-template <int D, int NW, bool MASK>
+// Few pairs: a pair's keys are cut into p.parts runs of p.part_keys keys, one
+// workgroup each (PART).  A part leaves its logits in attn_weights and
+// (max, sum, exp-weighted V sum) here; dense_merge_kernel combines the parts
+// and turns the logits into probabilities.  Static, so that the entry point
+// (which has no workspace argument) allocates nothing; launch_dense_dma holds
+// a lock over the two launches, and the null stream orders them.
+constexpr int kDenseParts = 16;       // parts of a pair
+constexpr int kDenseMaxParts = 1024;  // workgroups of a split launch
+__device__ float g_dense_acc[kDenseMaxParts * 128];
+__device__ float2 g_dense_ml[kDenseMaxParts];
+
+template <int D, int NW, bool MASK, bool PART>
 __global__ __launch_bounds__(NW * 64) void dense_attention_dma_kernel(DenseParams p) {
     using C = DenseDma<D, NW, MASK>;
     typedef float f4 __attribute__((ext_vector_type(4)));
     constexpr int EQ = D / 4, NQ = EQ / 4;
     extern __shared__ __attribute__((aligned(16))) char smem[];
-    const int64_t bh = blockIdx.x;
-    const int S = p.kv_len;
+    // the pair's keys s0 .. s0 + S - 1
+    const int64_t bh = PART ? blockIdx.x / p.parts : blockIdx.x;
+    const int s0 = PART ? ((int)blockIdx.x - (int)bh * p.parts) * p.part_keys : 0;
+    const int S = PART ? min(p.part_keys, p.kv_len - s0) : p.kv_len;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int qq = lane & 3, r = lane >> 2;
-    const char* kb = reinterpret_cast<const char*>(p.k + bh * D * S);
-    const char* vb = reinterpret_cast<const char*>(p.v + bh * D * S);
+    const char* kb = reinterpret_cast<const char*>(p.k + (bh * p.kv_len + s0) * D);
+    const char* vb = reinterpret_cast<const char*>(p.v + (bh * p.kv_len + s0) * D);
     const int64_t bytes = (int64_t)S * C::ROWB;
     const uint32_t wbase = (uint32_t)(uintptr_t)smem + wave * C::WAVE;
     const int nch = (S + 15) >> 4;
@@ -246,7 +262,7 @@ __global__ __launch_bounds__(NW * 64) void dense_attention_dma_kernel(DenseParam
     // segment flush.
     const int nit = (nch + NW - 1) / NW;
     float* logit = reinterpret_cast<float*>(smem + C::OFF_LOGIT);
-    float* wout = p.attn_weights + bh * S;
+    float* wout = p.attn_weights + bh * p.kv_len + s0;
 
     const float* q = p.q + bh * D * p.q_len;
     f4 qv[NQ];
@@ -277,7 +293,7 @@ __global__ __launch_bounds__(NW * 64) void dense_attention_dma_kernel(DenseParam
         }
         if constexpr (MASK) {  // lanes 0-15: the chunk's mask values
             const int s = 16 * c + lane;
-            dense_dma4(lane < 16 && s < S ? (const void*)(p.mask + s) : (const void*)kDenseZero16, sb + 2 * C::CH);
+            dense_dma4(lane < 16 && s < S ? (const void*)(p.mask + s0 + s) : (const void*)kDenseZero16, sb + 2 * C::CH);
         }
     };
 #pragma unroll
@@ -373,23 +389,102 @@ __global__ __launch_bounds__(NW * 64) void dense_attention_dma_kernel(DenseParam
         fw[w] = mw == -__builtin_inff() ? 0.0f : expf(mw - gm);
         total += red[NW * D + NW + w] * fw[w];
     }
-    const float inv = 1.0f / (total + 1e-9f);
+    const float inv = PART ? 1.0f : 1.0f / (total + 1e-9f);
+    float* out = PART ? g_dense_acc + (int64_t)blockIdx.x * D : p.out + bh * D;
     for (int d = threadIdx.x; d < D; d += NW * 64) {
         float o = 0.0f;
 #pragma unroll
         for (int w = 0; w < NW; ++w) o += red[w * D + d] * fw[w];
-        p.out[bh * D + d] = o * inv;
+        out[d] = o * inv;
     }
+    if (PART && threadIdx.x == 0) g_dense_ml[blockIdx.x] = make_float2(gm, total);
     // Probabilities: the last segment's logits from LDS, earlier ones from
     // attn_weights (written above by this same thread: the same index map).
     const int last0 = ((S - 1) / C::MAXS) * C::MAXS;
+    if constexpr (PART) {
+        for (int s = last0 + threadIdx.x; s < S; s += NW * 64) wout[s] = logit[s - last0];
+        return;
+    }
     for (int s = threadIdx.x; s < S; s += NW * 64) {
         const float l = s >= last0 ? logit[s - last0] : wout[s];
         wout[s] = expf(l - gm) * inv;
     }
 }
 
-template <int D, bool MASK>
+// Parts of a split pair -> out, and its logits -> probabilities: grid (pair,
+// run of kMergeKeys keys), every workgroup forming the pair's max and sum
+// from its parts.
+constexpr int kMergeKeys = 2048;
+
+template <int D>
+__global__ __launch_bounds__(kThreads) void dense_merge_kernel(DenseParams p) {
+    const int64_t bh = blockIdx.x;
+    const float2* ml = g_dense_ml + bh * p.parts;
+    float* w = p.attn_weights + bh * p.kv_len;
+    const int lo = blockIdx.y * kMergeKeys, hi = min(lo + kMergeKeys, p.kv_len);
+    float l[kMergeKeys / kThreads];
+#pragma unroll
+    for (int i = 0; i < kMergeKeys / kThreads; ++i) {
+        const int s = lo + i * kThreads + threadIdx.x;
+        l[i] = s < hi ? w[s] : 0.0f;
+    }
+    // every part's loads issued together (unused slots repeat part 0, weight 0)
+    const int d = threadIdx.x < D ? threadIdx.x : 0;
+    float2 x[kDenseParts];
+    float a[kDenseParts];
+#pragma unroll
+    for (int z = 0; z < kDenseParts; ++z) {
+        x[z] = ml[z < p.parts ? z : 0];
+        a[z] = g_dense_acc[(bh * p.parts + (z < p.parts ? z : 0)) * D + d];
+    }
+    float gm = x[0].x;
+#pragma unroll
+    for (int z = 1; z < kDenseParts; ++z) gm = fmaxf(gm, x[z].x);
+    float total = 0.0f, o = 0.0f;
+#pragma unroll
+    for (int z = 0; z < kDenseParts; ++z) {
+        if (z < p.parts) {
+            const float f = x[z].x == -__builtin_inff() ? 0.0f : expf(x[z].x - gm);
+            total += x[z].y * f;
+            o += a[z] * f;
+        }
+    }
+    const float inv = 1.0f / (total + 1e-9f);
+    if (blockIdx.y == 0 && threadIdx.x < D) p.out[bh * D + threadIdx.x] = o * inv;
+#pragma unroll
+    for (int i = 0; i < kMergeKeys / kThreads; ++i) {
+        const int s = lo + i * kThreads + threadIdx.x;
+        if (s < hi) w[s] = expf(l[i] - gm) * inv;
+    }
+}
+
+// Compute units of the current device (256 when it cannot be asked).
+int dense_cus() {
+    int dev = 0, n = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
+        return 256;
+    return n;
+}
+
+std::mutex g_dense_mu;  // the split's two launches: they share the scratch
+
+// Parts of each pair's keys (1: unsplit).  One workgroup per CU is resident
+// and reads at most about 50 GB/s, so pairs that leave CUs idle are split up
+// to one part per CU, at least 128 keys each, where the time that saves is
+// more than the second launch's 4.5 us: K and V of 512 KiB a pair for four
+// parts or more, 1.5 MiB for two or three.  Measured (us, unsplit / split):
+// 64 pairs x 4096 keys of 128 88.7 / 50.9, 64 x 1024 of 80 18.8 / 16.1;
+// 128 x 1024 of 128 30.0 / 30.5 (not split).  A second round of at most half
+// the CUs is also worth splitting for: 320 x 4096 of 128 249.6 / 214.9.
+int dense_parts(const DenseParams& p, int cus) {
+    const int64_t pairs = (int64_t)p.batch * p.heads, bytes = (int64_t)p.kv_len * p.head_dim * 8;
+    if (pairs > cus) return 2 * pairs <= 3 * (int64_t)cus && bytes >= (2 << 20) ? 3 : 1;
+    const int64_t z = std::min<int64_t>({cus / pairs, kDenseParts, p.kv_len / 128});
+    return z >= 2 && bytes >= (z >= 4 ? 512 << 10 : 1536 << 10) ? (int)z : 1;
+}
+
+template <int D, bool MASK, bool PART>
 hipError_t launch_dense_dma(const DenseParams& p, hipStream_t stream) {
     constexpr int NW = VCPP_DENSE_NW;
     using C = DenseDma<D, NW, MASK>;
@@ -398,19 +493,39 @@ hipError_t launch_dense_dma(const DenseParams& p, hipStream_t stream) {
     static bool attr_set[64] = {};
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64 || !attr_set[dev]) {
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(dense_attention_dma_kernel<D, NW, MASK>),
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(dense_attention_dma_kernel<D, NW, MASK, PART>),
                                                  hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS);
         if (e != hipSuccess) return e;
         if (dev >= 0 && dev < 64) attr_set[dev] = true;
     }
-    hipLaunchKernelGGL((dense_attention_dma_kernel<D, NW, MASK>), dim3(p.batch * p.heads), dim3(NW * 64), C::LDS,
-                       stream, p);
-    return hipGetLastError();
+    const int pairs = p.batch * p.heads;
+    hipLaunchKernelGGL((dense_attention_dma_kernel<D, NW, MASK, PART>), dim3(PART ? pairs * p.parts : pairs),
+                       dim3(NW * 64), C::LDS, stream, p);
+    hipError_t e = hipGetLastError();
+    if (PART && e == hipSuccess) {
+        hipLaunchKernelGGL((dense_merge_kernel<D>), dim3(pairs, (p.kv_len + kMergeKeys - 1) / kMergeKeys),
+                           dim3(kThreads), 0, stream, p);
+        e = hipGetLastError();
+    }
+    return e;
 }
 
 template <int D>
-hipError_t launch_dense_dma(const DenseParams& p, hipStream_t stream) {
-    return p.mask ? launch_dense_dma<D, true>(p, stream) : launch_dense_dma<D, false>(p, stream);
+hipError_t launch_dense_dma(const DenseParams& p0, hipStream_t stream) {
+    DenseParams p = p0;
+    // never more workgroups than the scratch has entries
+    const int64_t most = kDenseMaxParts / ((int64_t)p.batch * p.heads);
+    const int z = (int)std::min<int64_t>({dense_parts(p, dense_cus()), most, kDenseParts});
+    if (z > 1 && p.kv_len <= 65535 * kMergeKeys) {  // (dense_merge_kernel's grid.y)
+        // whole 64-key rounds of the four waves per part; every part holds a key
+        p.part_keys = ((p.kv_len + z - 1) / z + 63) / 64 * 64;
+        p.parts = (p.kv_len + p.part_keys - 1) / p.part_keys;
+        if (p.parts > 1) {
+            std::lock_guard<std::mutex> lock(g_dense_mu);
+            return p.mask ? launch_dense_dma<D, true, true>(p, stream) : launch_dense_dma<D, false, true>(p, stream);
+        }
+    }
+    return p.mask ? launch_dense_dma<D, true, false>(p, stream) : launch_dense_dma<D, false, false>(p, stream);
 }
 
 }  // namespace

@@ -70,6 +70,19 @@ def test_head_shapes(cuda, H, Hkv):
     _check(O.ORC_I8, [90] * 30 + [2600] * 3, H, Hkv, 64, 5400 + H)
 
 
+@pytest.mark.parametrize("n", [1, 7, 8, 9, 17])
+@pytest.mark.parametrize("H,Hkv", [(6, 1), (12, 3), (64, 8)])
+def test_workgroup_order(cuda, n, H, Hkv):
+    """(sequence, partition) counts around the rounds of eight XCDs."""
+    _check(O.ORC_F16, [200 + i for i in range(n)], H, Hkv, 80, 5450 + n)      # one partition
+    _check(O.ORC_F16, [700 - 90 * (i % 5) for i in range(n)], H, Hkv, 80, 5470 + n)
+
+
+def test_one_long_sequence(cuda):
+    """Over 128 partitions of 64 and 128 tokens: the rule takes longer ones."""
+    _check(O.ORC_F16, [33001], 12, 2, 128, 5490)
+
+
 @pytest.mark.parametrize("kind", KINDS)
 def test_skips(cuda, kind):
     """Short tables, missing and out-of-pool blocks, a length past the bound."""

@@ -165,13 +165,17 @@ struct DecodePlan {
 // 64 x 4096 at 1024, 51.0 against 61.0.  Up to 256 tokens one partition wins
 // outright (no merge: 4 x 256, 8.5 us against 9.4 at 64); up to 512 it does
 // where 64-token partitions would be too many (16 x 512, 14.0 against 14.5).
+// More than 128 partitions cost the merge more than the shorter ones save (1 x
+// 32768 with 12/2 heads of 128: 18.6 us at 128 tokens, 15.0 at 256).
 int32_t small_partition(int64_t units, int32_t max_ctx, bool page_mode) {
-    const int64_t most = 2 * (int64_t)device_cus();
-    if (units > most || units > 65535) return 0;
+    const int64_t most = std::min<int64_t>(2 * device_cus(), 1000);  // (decode.hip's kSeqsShift)
+    if (units > most) return 0;
     if (max_ctx <= 256) return 256;
     const int32_t top = page_mode ? 512 : 1024;
-    for (int32_t P = 64; P <= top; P *= 2)
-        if (units * num_parts(max_ctx, P) <= most) return max_ctx <= 512 && P > 64 ? 512 : P;
+    for (int32_t P = 64; P <= top; P *= 2) {
+        const int32_t parts = num_parts(max_ctx, P);
+        if (units * parts <= most && (parts <= 128 || P == top)) return max_ctx <= 512 && P > 64 ? 512 : P;
+    }
     return 0;
 }
 

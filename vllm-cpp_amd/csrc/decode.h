@@ -55,6 +55,7 @@ struct DecodeParams {
     float scale_log2;  // log2(e) / sqrt(head_dim)
     int32_t pipeline;  // fp16/int8 pipeline shape (tuning; 0 = default)
     int32_t small;     // fp16/int8/fp8: decode_small_kernel over fixed partitions
+    uint32_t seqs_magic;  // small: set by its launch
     int32_t page_mode; // fp16/int8, Hkv 8: 8-wave workgroups staging whole tiles in LDS
     int32_t page_grid; // workgroups that walk the num_wg ranges (page mode: a run each; else num_wg)
     // Balanced page split (one range per workgroup), g1 > 0: ranges of

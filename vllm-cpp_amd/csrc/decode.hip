@@ -749,7 +749,17 @@ void decode_mfma_kernel(DecodeParams p) {
 // 32/8 heads of 128, uniform contexts of half the maximum and up): 4 x 128
 // 6.6 against 17.7, 4 x 1024 11.7 against 17.8, 16 x 1024 18.7 against 23.7,
 // 16 x 2048 28.4 against 33.4; the rule is plan_decode's.
+// Rows that head slices do not cut at 128-byte lines were read 1.6 times
+// (head_dim 80) where a row's slices went to eight XCDs: a partition's slots on
+// one XCD take 32768 tokens (64/8 heads of 80) from 26.9 to 21.3 us, on int8
+// pages from 24.0 to 20.8, 60 sequences of up to 300 tokens from 13.0 to 11.3.
+// Aligned slices stay spread (four layers of 3 sequences up to 1200 tokens,
+// 32/8 heads of 128: 56.0 us against 57.9 on one XCD).
 constexpr int kSmallWaves = 4;
+constexpr int kXcds = 8;  // the dispatcher hands consecutive workgroups to consecutive XCDs
+// sp / num_seqs as a product with ceil(2^22 / num_seqs): exact for sp < 1024
+// (plan_decode's rule: two workgroups per CU).
+constexpr int kSeqsShift = 22;
 
 template <int KV, int D>
 __global__ __launch_bounds__(kSmallWaves * 64) __attribute__((amdgpu_waves_per_eu(4, 4)))
@@ -760,7 +770,9 @@ void decode_small_kernel(DecodeParams p) {
     __shared__ float2 ml_s[W][8];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int g = lane >> 4, c = lane & 15;
-    const int s = blockIdx.x, pair = blockIdx.y, part = blockIdx.z;
+    const int pair = blockIdx.y, sp = blockIdx.z * gridDim.x + blockIdx.x;
+    const int part = (uint32_t)sp * p.seqs_magic >> kSeqsShift, s = sp - part * p.num_seqs;
+    if (part >= p.max_parts) return;  // whole workgroup (the last round's rest)
     const int kvh = pair / p.qchunks, qc = pair - kvh * p.qchunks;
     const int head_base = kvh * p.group + qc * 8;
     const int gc = min(8, p.group - qc * 8);
@@ -1894,8 +1906,15 @@ hipError_t launch_merge_parts(const DecodeParams& p, hipStream_t stream) {
 }
 
 template <int KV>
-hipError_t launch_small(const DecodeParams& p, hipStream_t stream) {
-    const dim3 grid(p.num_seqs, p.pairs, p.max_parts), block(kSmallWaves * 64);
+hipError_t launch_small(const DecodeParams& p0, hipStream_t stream) {
+    DecodeParams p = p0;
+    p.seqs_magic = ((1u << kSeqsShift) + p.num_seqs - 1) / p.num_seqs;
+    const int sp = p.num_seqs * p.max_parts;
+    // Workgroup ids go round the XCDs.  Where a row's slices share cache lines
+    // they go to one XCD, whose L2 then serves the line's second reader.
+    const bool shared = p.head_dim * (KV == VCPP_KV_F16 ? 2 : 1) % 128 != 0;
+    const int gx = shared ? kXcds : p.num_seqs;
+    const dim3 grid(gx, p.pairs, (sp + gx - 1) / gx), block(kSmallWaves * 64);
     switch (p.head_dim) {
         case 64: hipLaunchKernelGGL((decode_small_kernel<KV, 64>), grid, block, 0, stream, p); break;
         case 80: hipLaunchKernelGGL((decode_small_kernel<KV, 80>), grid, block, 0, stream, p); break;

@@ -113,3 +113,16 @@ def test_block_sizes(cuda):
         outs.append(out.cpu().numpy())
     assert np.array_equal(outs[0], outs[1]) and np.array_equal(outs[0], outs[2])
     assert np.isfinite(outs[0]).all()
+
+
+def test_int8_small_scales(cuda):
+    """V scales near 2^-11: P times a scale keeps its 22 bits (about 2e-7
+    here with fp32 sums of 300 terms; low parts lost to fp16's subnormals
+    would show 3e-5)."""
+    ctx = np.array([300, 41, 256], dtype=np.int32)
+    pool = O.make_pool(O.ORC_I8, 5800, 64, 8, 80, 0.0, 0.02)
+    q = O.normal(5801, (3, 64, 80))
+    tables, _ = _tables(5802, ctx, 64, O.BS)
+    want = O.decode(pool, q, tables, ctx, 64)
+    got = gpu_decode(DevPool(pool), q, tables, ctx, 64)
+    assert np.linalg.norm(got - want) <= 3e-6 * np.linalg.norm(want)

@@ -419,6 +419,11 @@ __device__ __forceinline__ void merge_unit(int nfr, int fw, int lane, bool act, 
     if (act) *reinterpret_cast<f4*>(out) = acc * (1.0f / (L + 1e-9f));
 }
 
+// P's low parts are held times 2^11, the size of their high parts: unscaled,
+// int8 pages' P (times a V scale of 2^-6 or so) leave low parts below fp16's
+// subnormal step of 2^-24.
+constexpr float kLoScale = 2048.0f;
+
 // One wave's attention of 8 query heads of a kv head over a list of 16-token
 // tiles of one sequence, K and V loaded straight from the pages into
 // registers.  The state is the online softmax (m_run, l_run per head column)
@@ -555,7 +560,7 @@ struct WaveAttn {
                         pr = pr > 0.f ? pr * h_to_f((r & 1) ? (wd >> 16) : (wd & 0xFFFFu)) : 0.f;
                     }
                     const _Float16 hi = (_Float16)pr;
-                    pa[r] = c < 8 ? hi : (_Float16)(pr - (float)hi);
+                    pa[r] = c < 8 ? hi : (_Float16)((pr - (float)hi) * kLoScale);
                 }
                 lds_char* vt = lds + j * kTile * D * 2;
 #pragma unroll
@@ -591,8 +596,8 @@ struct WaveAttn {
         }
     }
 
-    // Per-head totals of this wave: O rows h (hi) + h + 8 (lo) summed in
-    // place (lane (g, c), g < 2: heads 4 g + r, columns 16 t + c), and the
+    // Per-head totals of this wave: O rows h (hi) + h + 8 (lo, kLoScale) summed
+    // in place (lane (g, c), g < 2: heads 4 g + r, columns 16 t + c), and the
     // heads' (max, sum) of those rows.
     __device__ __forceinline__ void finish(int g, float (&mh)[4], float (&lh)[4]) {
         float lt = l_run;
@@ -601,7 +606,7 @@ struct WaveAttn {
 #pragma unroll
         for (int t = 0; t < NT; ++t)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) o[t][r] += shfl_xor(o[t][r], 32);
+            for (int r = 0; r < 4; ++r) o[t][r] = fmaf(shfl_xor(o[t][r], 32), 1.0f / kLoScale, o[t][r]);
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             lh[r] = shfl(lt, (4 * g + r) & 7);

@@ -1,8 +1,8 @@
 """The C-ABI entry points under HIP graph capture (torch.cuda.graph): a
 captured vcpp_paged_decode, vcpp_paged_prefill_split and
-vcpp_paged_mixed_step (whose decode merge forks onto a side stream and joins
-back by events) replay bit-identically to the eager calls, three replays in
-a row with eager work on the outputs between them.  The kernels' split and
+vcpp_paged_mixed_step (decode, its merge and the prefill, one after the
+other) replay bit-identically to the eager calls, three replays in a row with
+eager work on the outputs between them.  The kernels' split and
 merge orders are fixed by the shapes, so eager and replayed results are
 bit-equal."""
 import pytest
@@ -104,10 +104,10 @@ def test_graph_replays_match_eager(cuda, which):
 
 def test_mixed_capture_beside_eager_stream(cuda):
     """One stream captures a mixed step while another stream of the same GPU
-    runs mixed steps eagerly inside the capture: each caller stream forks its
-    merge onto its own side stream, so the eager steps are neither recorded
-    into the graph nor break the capture, and both results match the eager
-    reference (the graph over three replays)."""
+    runs mixed steps eagerly inside the capture: a step stays on its caller's
+    stream, so the eager steps are neither recorded into the graph nor break
+    the capture, and both results match the eager reference (the graph over
+    three replays)."""
     wa = setup(97)
     wb = setup(98)
     wsa = workspace(wa, "mixed")
@@ -125,7 +125,7 @@ def test_mixed_capture_beside_eager_stream(cuda):
                                 wb["pout"], wb["ptab"], wb["q_start"], wb["prefix"], wb["max_chunk"], H,
                                 workspace=wsb, stream=sb)
 
-    mixed_b()  # its side stream exists before the capture
+    mixed_b()
     torch.cuda.synchronize()
     for o in ("dout", "pout"):
         wb[o].fill_(float("nan"))
@@ -149,3 +149,25 @@ def test_mixed_capture_beside_eager_stream(cuda):
             assert torch.equal(wa[o], ref_a[o]), "replay %d: %s differs" % (rep, o)
             # nothing of stream b's step was recorded into the graph
             assert torch.isnan(wb[o]).all(), "replay %d wrote stream b's %s" % (rep, o)
+
+
+def test_mixed_step_is_one_chain(cuda):
+    """A captured mixed step is three kernels in a row: nothing beside the
+    prefill takes CUs from its tiles, no events between streams."""
+    import ctypes
+    hip = ctypes.CDLL(next(l.split()[-1] for l in open("/proc/self/maps") if "libamdhip64" in l))
+    w = setup(99)
+    ws = workspace(w, "mixed")
+    mixed(w, ws)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph):
+        mixed(w, ws)
+    raw, n = ctypes.c_void_p(graph.raw_cuda_graph()), ctypes.c_size_t()
+    assert hip.hipGraphGetNodes(raw, None, ctypes.byref(n)) == 0
+    assert n.value == 3
+    assert hip.hipGraphGetEdges(raw, None, None, ctypes.byref(n)) == 0
+    assert n.value == 2
+    a, b = (ctypes.c_void_p * 2)(), (ctypes.c_void_p * 2)()
+    assert hip.hipGraphGetEdges(raw, a, b, ctypes.byref(n)) == 0
+    assert len(set(a)) == 2 and len(set(b)) == 2, "a node has two successors"

@@ -11,7 +11,6 @@
 #include <algorithm>
 #include <cstdio>
 #include <cstdlib>
-#include <map>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -97,50 +96,6 @@ int device_cus() {
         cus[dev] = n;
     }
     return cus[dev];
-}
-
-// The mixed step's side streams (default priority) and fork / join events:
-// one set per (device, caller stream), made on first use and kept for the
-// process.  Each caller stream forks onto its own side stream, so steps on
-// different streams never share one (a side stream joined to one stream's
-// graph capture is never used by another stream meanwhile).  Calls on one
-// stream are serialised by the caller, as for every entry point; g_fork_mu
-// guards only the table.
-std::mutex g_fork_mu;
-
-const vcpp::MergeFork* merge_fork(hipStream_t stream) {
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0) return nullptr;
-    // Only for a stream of the current device (the side stream is made there).
-    hipDevice_t sdev = -1;
-    if (stream && (hipStreamGetDevice(stream, &sdev) != hipSuccess || sdev != dev)) {
-        (void)hipGetLastError();
-        return nullptr;
-    }
-    struct Entry {
-        vcpp::MergeFork mf;
-        bool ok;
-    };
-    static std::map<std::pair<int, hipStream_t>, Entry> table;
-    std::lock_guard<std::mutex> lock(g_fork_mu);
-    auto it = table.find({dev, stream});
-    if (it == table.end()) {
-        Entry en{};
-        bool ok = hipStreamCreateWithFlags(&en.mf.side, hipStreamNonBlocking) == hipSuccess;
-        ok = ok && hipEventCreateWithFlags(&en.mf.fork, hipEventDisableTiming) == hipSuccess;
-        ok = ok && hipEventCreateWithFlags(&en.mf.join, hipEventDisableTiming) == hipSuccess;
-        if (!ok) (void)hipGetLastError();
-        en.ok = ok;
-        it = table.emplace(std::make_pair(dev, stream), en).first;
-    }
-    return it->second.ok ? &it->second.mf : nullptr;
-}
-
-// VCPP_NO_MERGE_FORK=1: the mixed step's merge stays on the caller's stream
-// (for measurement).
-bool no_merge_fork() {
-    const char* e = std::getenv("VCPP_NO_MERGE_FORK");
-    return e && e[0] == '1';
 }
 
 // Launch geometry and workspace layout of one decode call.
@@ -776,44 +731,33 @@ int vcpp_paged_mixed_step(const vcpp_kv_pages* kv, const float* dq, float* dout,
     if (rc != VCPP_OK) return rc;
     const bool has_p = num_chunks > 0 && max_chunk_len > 0;
     const int32_t fg = num_seqs > 0 && has_p ? mixed_grid(kv, num_heads, p_max_blocks_per_seq) : 0;
-    if (fg == 0 && num_seqs > 0 && has_p && kv->dtype != VCPP_KV_F32 && !no_merge_fork()) {
-        // Decode, then the prefill on the caller's stream, with the decode's
-        // merge on a side stream between them (it depends on the decode
-        // only, and overlaps the prefill); the caller's stream waits for it
-        // at the end.
-        const DecodePlan pl = plan_decode(kv, num_seqs, num_heads, max_context_len, 0);
-        if (pl.max_parts > 65535) return fail(VCPP_E_UNSUPPORTED, "too many partitions (%d)", pl.max_parts);
-        rc = check_workspace(pl, workspace, workspace_bytes);
-        if (rc != VCPP_OK) return rc;
-        const vcpp::DecodeParams dp = decode_params(kv, dq, dout, d_block_tables, d_max_blocks_per_seq,
-                                                    d_table_lens, d_context_lens, num_seqs, max_context_len,
-                                                    num_heads, 0, pl, workspace);
-        const vcpp::PrefillParams pp = prefill_params(kv, pq, pout, p_block_tables, p_max_blocks_per_seq,
-                                                      q_start, prefix_lens, num_chunks, max_chunk_len, num_heads);
+    if (fg == 0) {
+        // Decode (with its merge), then prefill, all on the caller's stream.
+        // The merge on a side stream beside the prefill costs more than the
+        // 4 to 5 us it hides: its workgroups take CUs before the prefill's
+        // tiles are placed in heavy-and-light pairs, and the two events cost
+        // short steps about 20 us.  In turn / merge forked: 128 int8 decodes
+        // up to 8192 tokens + 4 x 512 rows 225.4 / 229.0 us; 4 fp16 decodes
+        // up to 1544 + 2 x 22 rows 20.2 / 49.4; no step of twenty was faster
+        // forked by more than 0.1 us.
         const hipStream_t s = static_cast<hipStream_t>(stream);
-        const vcpp::MergeFork* mf = merge_fork(s);
-        bool forked = false;
-        hipError_t e = vcpp::launch_decode(dp, s, mf, &forked);
-        // Once the merge is forked, the caller's stream joins it whatever
-        // fails later, so the stream stays ordered after the merge (and a
-        // capture ends with the side stream joined).
-        const hipError_t ep = e == hipSuccess ? vcpp::launch_prefill(pp, s) : hipSuccess;
-        const hipError_t ej = forked ? hipStreamWaitEvent(s, mf->join, 0) : hipSuccess;
-        if (e != hipSuccess) return hip_fail(e, "decode launch");
-        if (ep != hipSuccess) return hip_fail(ep, "prefill launch");
-        if (ej != hipSuccess) return hip_fail(ej, "merge join");
-        return VCPP_OK;
-    }
-    if (fg == 0) {  // two launches on the stream: decode, then prefill
         if (num_seqs > 0) {
-            rc = vcpp_paged_decode(kv, dq, dout, d_block_tables, d_max_blocks_per_seq, d_table_lens,
-                                   d_context_lens, num_seqs, max_context_len, num_heads, 0, workspace,
-                                   workspace_bytes, stream);
+            const DecodePlan pl = plan_decode(kv, num_seqs, num_heads, max_context_len, 0);
+            if (pl.max_parts > 65535) return fail(VCPP_E_UNSUPPORTED, "too many partitions (%d)", pl.max_parts);
+            rc = check_workspace(pl, workspace, workspace_bytes);
             if (rc != VCPP_OK) return rc;
+            const vcpp::DecodeParams dp = decode_params(kv, dq, dout, d_block_tables, d_max_blocks_per_seq,
+                                                        d_table_lens, d_context_lens, num_seqs, max_context_len,
+                                                        num_heads, 0, pl, workspace);
+            const hipError_t e = vcpp::launch_decode(dp, s);
+            if (e != hipSuccess) return hip_fail(e, "decode launch");
         }
         if (!has_p) return VCPP_OK;
-        return vcpp_paged_prefill(kv, pq, pout, p_block_tables, p_max_blocks_per_seq, q_start, prefix_lens,
-                                  num_chunks, max_chunk_len, num_heads, stream);
+        const vcpp::PrefillParams pp = prefill_params(kv, pq, pout, p_block_tables, p_max_blocks_per_seq,
+                                                      q_start, prefix_lens, num_chunks, max_chunk_len, num_heads);
+        const hipError_t e = vcpp::launch_prefill(pp, s);
+        if (e != hipSuccess) return hip_fail(e, "prefill launch");
+        return VCPP_OK;
     }
     const DecodePlan pl = plan_decode(kv, num_seqs, num_heads, max_context_len, 0, fg);
     rc = check_workspace(pl, workspace, workspace_bytes);

@@ -1936,7 +1936,7 @@ int decode_group_count(int pairs) {
     return (pairs + wpw - 1) / wpw;
 }
 
-hipError_t launch_decode(const DecodeParams& p, hipStream_t stream, const MergeFork* mf, bool* forked) {
+hipError_t launch_decode(const DecodeParams& p, hipStream_t stream) {
     if (p.num_seqs == 0) return hipSuccess;
     hipError_t err;
     const bool prof = prof_enabled();
@@ -1996,20 +1996,9 @@ hipError_t launch_decode(const DecodeParams& p, hipStream_t stream, const MergeF
     if (err != hipSuccess) return err;
     if (prof) prof_end(kKernelDecode, stream);
     if (p.small && p.max_parts == 1) return hipSuccess;  // finished in place
-    if (mf) {
-        err = hipEventRecord(mf->fork, stream);
-        if (err == hipSuccess) err = hipStreamWaitEvent(mf->side, mf->fork, 0);
-        if (err != hipSuccess) return err;
-        if (forked) *forked = true;
-        stream = mf->side;
-    }
     if (prof) prof_begin(kKernelMerge, stream);
     err = p.small ? launch_merge_parts(p, stream) : launch_merge_split(p, stream);
     if (prof) prof_end(kKernelMerge, stream);
-    if (mf) {  // recorded even after a failed merge launch, so the caller can always join
-        const hipError_t ej = hipEventRecord(mf->join, stream);
-        if (err == hipSuccess) err = ej;
-    }
     return err;
 }
 

@@ -197,6 +197,10 @@ int vcpp_paged_prefill(const vcpp_kv_pages* kv, const uint16_t* q, float* out,
  *   max_prefix_len  host-side upper bound of prefix_lens (sizes the split)
  *   workspace       device scratch of at least vcpp_prefill_workspace_size(...)
  *                   bytes, 16-byte aligned (none needed when that is 0)
+ * That size is of the call's own arguments and not monotonic in them (a longer
+ * chunk fills the GPU with fewer parts, and with none at some length).  One
+ * buffer for calls of any size: no call needs more than 1024 * compute units *
+ * (4 * head_dim + 8) + 256 bytes (half of that at head_dim 128).
  * Calls on one stream may share a workspace; calls that overlap may not.
  * No reference counterpart: the reference prefills one position at a time
  * (src/paged_engine.cpp:381-384).

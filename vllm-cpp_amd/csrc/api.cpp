@@ -628,34 +628,52 @@ int vcpp_paged_prefill(const vcpp_kv_pages* kv, const uint16_t* q, float* out,
     return VCPP_OK;
 }
 
-// Key parts of a split prefill: up to enough workgroups to fill two per CU,
-// each part at least 16 key blocks (512 keys) of the longest chunk, at most
-// 16; of those the count that a sum of the launch's rounds puts first.  In
-// units of one 32-key block of two resident workgroups per CU (about 1.3 us):
-// a round of a part's blocks, 0.65 of that where the last round leaves one
-// workgroup per CU, 5 for a round's start and end, and the partials' traffic.
-// The fullest count is not it where it spills a few workgroups into a round
-// of their own: 48 tiles in 11 parts are 528 workgroups, 56.0 us for three
-// 40-token chunks on 7000-token prefixes (32/8 heads of 128), 41.9 in 10
-// parts; one 300-token chunk on 16384, 146.9 in 7 parts, 111.8 in 6.  But
-// 384 tiles (three 500-token chunks on 8192, 64/8 heads of 80) take 365 us
-// whole and 325 in two parts.
-static int32_t prefill_splits(const vcpp_kv_pages* kv, int32_t num_chunks, int32_t max_chunk_len,
-                              int32_t max_prefix_len, int32_t num_heads) {
-    if (num_chunks <= 0 || max_chunk_len <= 0 || max_prefix_len < 0) return 1;
+// Workgroups of an unsplit prefill call.
+static int64_t prefill_items(const vcpp_kv_pages* kv, int32_t num_chunks, int32_t max_chunk_len, int32_t num_heads) {
     const int64_t qt = kv->head_dim <= 80 ? 64 : 32;  // query rows per workgroup
-    const int64_t items = (max_chunk_len + qt - 1) / qt * num_chunks * kv->num_kv_heads *
-                          vcpp::prefill_head_groups(num_heads / kv->num_kv_heads);
-    const int64_t cus = device_cus(), slots = 2 * cus;
+    return (max_chunk_len + qt - 1) / qt * num_chunks * kv->num_kv_heads *
+           vcpp::prefill_head_groups(num_heads / kv->num_kv_heads);
+}
+
+// Most key parts a split prefill call is cut into, and what its workspace is
+// sized for: enough workgroups to fill two per CU, each part at least 16 key
+// blocks (512 keys) of the longest chunk, at most 16.  The rows times parts of
+// this count change little with the call's rows, so that a buffer sized for a
+// longer call mostly holds a shorter one's partials; those of prefill_splits'
+// own count jump (three chunks on 2000-token prefixes, 64/8 heads of 64: one
+// part at 512 rows, two at 320).
+static int32_t prefill_most_splits(const vcpp_kv_pages* kv, int32_t num_chunks, int32_t max_chunk_len,
+                                   int32_t max_prefix_len, int32_t num_heads) {
+    if (num_chunks <= 0 || max_chunk_len <= 0 || max_prefix_len < 0) return 1;
+    const int64_t items = prefill_items(kv, num_chunks, max_chunk_len, num_heads);
+    const int64_t slots = 2 * (int64_t)device_cus();
     if (items >= slots) return 1;
     const int64_t want = (slots + items - 1) / items;
     const int64_t by_len = ((int64_t)max_prefix_len + max_chunk_len) / (16 * 32);
-    const int64_t most = std::min<int64_t>({want, by_len, (int64_t)vcpp::kMaxPrefillSplits});
+    return (int32_t)std::max<int64_t>(1, std::min<int64_t>({want, by_len, (int64_t)vcpp::kMaxPrefillSplits}));
+}
+
+// Key parts of a split prefill: of 1 .. prefill_most_splits the count that a
+// sum of the launch's rounds puts first.  In units of one 32-key block of two
+// resident workgroups per CU (about 1.3 us): a round of a part's blocks, 0.65
+// of that where the last round leaves one workgroup per CU, 5 for a round's
+// start and end, and the partials' traffic.  The fullest count is not it where
+// it spills a few workgroups into a round of their own: 48 tiles in 11 parts
+// are 528 workgroups, 56.0 us for three 40-token chunks on 7000-token prefixes
+// (32/8 heads of 128), 41.9 in 10 parts; one 300-token chunk on 16384, 146.9
+// in 7 parts, 111.8 in 6.  But 384 tiles (three 500-token chunks on 8192, 64/8
+// heads of 80) take 365 us whole and 325 in two parts.
+static int32_t prefill_splits(const vcpp_kv_pages* kv, int32_t num_chunks, int32_t max_chunk_len,
+                              int32_t max_prefix_len, int32_t num_heads) {
+    const int32_t most = prefill_most_splits(kv, num_chunks, max_chunk_len, max_prefix_len, num_heads);
+    if (most == 1) return 1;
+    const int64_t items = prefill_items(kv, num_chunks, max_chunk_len, num_heads);
+    const int64_t cus = device_cus(), slots = 2 * cus;
     const double blocks = ((double)max_prefix_len + max_chunk_len) / 32;
     const double part_bytes = 8.0 * num_chunks * max_chunk_len * num_heads * kv->head_dim;  // written and read
     int32_t best = 1;
     double best_cost = 0;
-    for (int32_t s = 1; s <= std::max<int64_t>(1, most); ++s) {
+    for (int32_t s = 1; s <= most; ++s) {
         const int64_t full = items * s / slots, rest = items * s % slots;
         const double cost = blocks / s * (full + (rest == 0 ? 0.0 : rest <= cus ? 0.65 : 1.0)) +
                             5.0 * (full + (rest > 0)) + (s > 1 ? s * part_bytes / 6.5e6 : 0.0);
@@ -670,7 +688,7 @@ static int32_t prefill_splits(const vcpp_kv_pages* kv, int32_t num_chunks, int32
 size_t vcpp_prefill_workspace_size(const vcpp_kv_pages* kv, int32_t num_chunks, int32_t max_chunk_len,
                                    int32_t max_prefix_len, int32_t num_heads) {
     if (!kv || kv->num_kv_heads <= 0 || num_heads <= 0 || num_heads % kv->num_kv_heads != 0) return 0;
-    const int32_t s = prefill_splits(kv, num_chunks, max_chunk_len, max_prefix_len, num_heads);
+    const int32_t s = prefill_most_splits(kv, num_chunks, max_chunk_len, max_prefix_len, num_heads);
     return vcpp::prefill_split_bytes(s, (int32_t)std::min<int64_t>((int64_t)num_chunks * max_chunk_len, INT32_MAX),
                                      num_heads, kv->head_dim);
 }

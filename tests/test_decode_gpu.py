@@ -272,8 +272,8 @@ def test_block_size_32(cuda):
 @pytest.mark.parametrize("partition", [0, 128])
 @pytest.mark.parametrize("D", [64, 128])
 def test_fp8_other_head_dims(cuda, D, partition):
-    """FP8 pages (the reference KV_FP8 pool's E4M3 bytes) on the page-staged
-    kernel (D 64) and the register-path kernel (D 128, fixed partitions)."""
+    """FP8 pages (the reference KV_FP8 pool's E4M3 bytes) on the small-batch
+    kernel (partition_size 0) and the page-staged one (fixed partitions)."""
     ctx = np.array([5, 48, 300, 1], dtype=np.int32)
     pool = O.make_pool(O.ORC_FP8, 231, 40, 8, D, std=3.0)
     q = O.normal(233, (4, 64, D))
@@ -290,7 +290,9 @@ def test_fp8_other_head_dims(cuda, D, partition):
 def test_page_kernel_shapes(cuda, kind, heads, D, partition):
     """Every page-staged kernel shape (8 kv heads per workgroup at head_dim 64
     and 80; 4 per workgroup for 4-head multiples and head_dim 128, walked as
-    head groups of one range) on ragged contexts, both split modes."""
+    head groups of one range) on ragged contexts in fixed partitions;
+    partition_size 0 runs the small-batch kernel on a batch of this size (the
+    balanced split: test_decode_balanced_gpu.py)."""
     H, Hkv = heads
     ctx = np.array([0, 5, 16, 31, 300, 1025, 777, 64, 2000, 1], dtype=np.int32)
     nb = int(sum((int(c) + O.BS - 1) // O.BS for c in ctx)) + 6

@@ -52,6 +52,18 @@ def test_split_merge(cuda, ctx, H, Hkv, D, partition):
     _run(O.ORC_F16, ctx, H, Hkv, D, partition, 4100 + D + H)
 
 
+@pytest.mark.parametrize("partition", [0, 64])
+@pytest.mark.parametrize("n,long,H,Hkv,D", [
+    (129, 3001, 64, 8, 80), (200, 700, 28, 4, 128), (450, 90, 12, 2, 128), (300, 5003, 8, 8, 64), (600, 2100, 20, 2, 64)])
+def test_split_merge_many(cuda, n, long, H, Hkv, D, partition):
+    """Many sequences, a workgroup per (sequence, kv-head slot): more lengths
+    than its waves scan in a round, empty ones among them, one sequence over
+    many ranges, slots of fewer units than waves."""
+    ctx = [(29 * i * i + 5) % 67 for i in range(n)]
+    ctx[n // 3] = long
+    _run(O.ORC_F16, ctx, H, Hkv, D, partition, 4200 + n)
+
+
 def test_split_merge_fp8(cuda):
     _run(O.ORC_FP8, SOME, 64, 8, 80, 0, 4300)
 

@@ -843,42 +843,29 @@ void decode_small_kernel(DecodeParams p) {
     }
 }
 
-// Sequences split over several ranges get their partial blocks merged;
-// everything else was finished in place.  A unit of work is 256 outputs of
-// one (sequence, kv-head slot): grid (sequence, 4 slots, slot of the 4 and
-// units / SL), SL units of FW waves per workgroup.
-template <int D, int SL, int FW>
-__global__ __launch_bounds__(SL * FW * 64) void merge_split_kernel(DecodeParams p) {
-    __shared__ float part[FW > 1 ? SL * FW : 1][64][6];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int fw = wave % FW, sl = wave / FW;
-    const int pair = 4 * blockIdx.y + (blockIdx.z & 3), unit = (blockIdx.z >> 2) * SL + sl;
-    const int s = blockIdx.x;
-    if (pair >= p.pairs) return;
-    const int G = p.num_wg, X = p.switch_tiles;
-    int T = 0, S = 0, K = 0, KS = 0;  // tiles and non-empty sequences: all, before s
-    for (int base = 0; base < p.num_seqs; base += 128) {
-        int nt[2];
-#pragma unroll
-        for (int k = 0; k < 2; ++k) {
-            const int i = base + 64 * k + lane;
-            nt[k] = i < p.num_seqs ? tiles_of(p, i) : 0;
-        }
-#pragma unroll
-        for (int k = 0; k < 2; ++k) {
-            const bool before = base + 64 * k + lane < s;
-            T += wave_sum(nt[k]);
-            S += wave_sum(before ? nt[k] : 0);
-            K += __builtin_popcountll(__ballot(nt[k] > 0));
-            KS += __builtin_popcountll(__ballot(before && nt[k] > 0));
-        }
+// Tiles and non-empty sequences of the batch: all of them (T, K) and those
+// before s (S, KS), 64 sequences (one per lane) an add.
+struct SplitSums {
+    int T = 0, S = 0, K = 0, KS = 0;
+    __device__ __forceinline__ void add(const DecodeParams& p, int s, int i) {
+        const int nt = i < p.num_seqs ? tiles_of(p, i) : 0;
+        const bool before = i < s;
+        T += wave_sum(nt);
+        S += wave_sum(before ? nt : 0);
+        K += __builtin_popcountll(__ballot(nt > 0));
+        KS += __builtin_popcountll(__ballot(before && nt > 0));
     }
-    const int E = S + tiles_of(p, s);
-    if (E <= S) return;  // no tiles: zeroed by the decode kernel
+};
+
+// One unit of the merge, outputs 256 unit .. + 255 of (sequence s of `mine` > 0
+// tiles, kv-head slot `pair`), by FW waves (this one fw).
+template <int D, int FW>
+__device__ __forceinline__ void merge_split_unit(const DecodeParams& p, const SplitSums& c, int mine, int s, int pair,
+                                                 int unit, int fw, int lane, float (*lds)[64][6]) {
     // the split's axis: tile t of s sits at t + X (non-empty sequences up to s)
-    const int Tv = T + X * K, shift = X * (KS + 1);
-    const Spans sp{Split(Tv, G, p.g1, p.g1_share), p.page_grid};
-    const int w0 = sp.span_of(S + shift), w1 = sp.span_of(E - 1 + shift);
+    const int X = p.switch_tiles, shift = X * (c.KS + 1);
+    const Spans sp{Split(c.T + X * c.K, p.num_wg, p.g1, p.g1_share), p.page_grid};
+    const int w0 = sp.span_of(c.S + shift), w1 = sp.span_of(c.S + mine - 1 + shift);
     if (w0 == w1) return;  // finished in place
     const int kvh = pair / p.qchunks, qc = pair - kvh * p.qchunks;
     const int n_out = min(8, p.group - qc * 8) * D;
@@ -890,7 +877,61 @@ __global__ __launch_bounds__(SL * FW * 64) void merge_split_kernel(DecodeParams 
     merge_unit<FW>(
         w1 - w0 + 1, fw, lane, act, out, [&](int i) { return all || sp.live(w0 + i); },
         [&](int i) { return p.ws_ml + frag_block(w0, i, p.pairs, pair) * 16 + h; },
-        [&](int i) { return p.ws_o + frag_block(w0, i, p.pairs, pair) * (8 * D) + ec; }, part + (FW > 1 ? sl * FW : 0));
+        [&](int i) { return p.ws_o + frag_block(w0, i, p.pairs, pair) * (8 * D) + ec; }, lds);
+}
+
+// Sequences split over several ranges get their partial blocks merged;
+// everything else was finished in place.  A unit of work is 256 outputs of
+// one (sequence, kv-head slot): grid (sequence, 4 slots, slot of the 4 and
+// unit), FW waves each.
+template <int D, int FW>
+__global__ __launch_bounds__(FW * 64) void merge_split_kernel(DecodeParams p) {
+    __shared__ float part[FW][64][6];
+    const int lane = threadIdx.x & 63;
+    const int pair = 4 * blockIdx.y + (blockIdx.z & 3);
+    const int s = blockIdx.x;
+    if (pair >= p.pairs) return;
+    SplitSums c;
+    for (int base = 0; base < p.num_seqs; base += 128) {
+        c.add(p, s, base + lane);
+        c.add(p, s, base + 64 + lane);
+    }
+    const int mine = tiles_of(p, s);
+    if (mine <= 0) return;  // no tiles: zeroed by the decode kernel
+    merge_split_unit<D, FW>(p, c, mine, s, pair, blockIdx.z >> 2, threadIdx.x >> 6, lane, part);
+}
+
+// The same for many units: grid (sequence, kv-head slot), one wave per unit of
+// the slot.  The scan of the lengths is most of what such a workgroup does
+// (most sequences of a large batch lie in one range or two), so its waves
+// share it.  With a scan per wave, three of them where one had covered a slot,
+// decode and merge of 1024 sequences up to 488 tokens (64/8 heads of 80) took
+// 181.3 us on fp16 and 137.7 on FP8 pages; they take 168.6 and 125.0.  More slots
+// to a workgroup share the scan further but put the units of a sequence of
+// many ranges on fewer CUs: 199 short sequences beside one of 65536 tokens
+// 78.2 us so (fp16), 82.0 with two slots, 90.3 with four.
+template <int D>
+__global__ __launch_bounds__((8 * D + 255) / 256 * 64) void merge_split_slot_kernel(DecodeParams p) {
+    constexpr int U = (8 * D + 255) / 256;
+    __shared__ int4 sums[U];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int s = blockIdx.x;
+    SplitSums c;
+    for (int base = 64 * wave; base < p.num_seqs; base += 64 * U) c.add(p, s, base + lane);
+    const int mine = tiles_of(p, s);
+    if (lane == 0) sums[wave] = make_int4(c.T, c.S, c.K, c.KS);
+    __syncthreads();
+    if (mine <= 0 || 256 * wave >= min(8, p.group) * D) return;  // no tiles: zeroed by the decode kernel
+    c = SplitSums();
+#pragma unroll
+    for (int w = 0; w < U; ++w) {
+        const int4 x = sums[w];
+        c.T += x.x;
+        c.S += x.y;
+        c.K += x.z;
+        c.KS += x.w;
+    }
+    merge_split_unit<D, 1>(p, c, mine, s, blockIdx.y, wave, 0, lane, nullptr);
 }
 
 // ---- fp32 pages -----------------------------------------------------------
@@ -1873,10 +1914,10 @@ hipError_t launch_mfma(const DecodeParams& p, hipStream_t stream) {
 // 128..4096, 1536 units of 4, 4.8 / 4.9 / 9.4.
 int merge_waves(int64_t units) { return units * 8 <= 2048 ? 8 : units * 2 <= 2048 ? 2 : 1; }
 
-template <int D, int SL, int FW>
+template <int D, int FW>
 hipError_t launch_merge_shape(const DecodeParams& p, int units, hipStream_t stream) {
-    const dim3 grid(p.num_seqs, (p.pairs + 3) / 4, (units + SL - 1) / SL * 4);
-    hipLaunchKernelGGL((merge_split_kernel<D, SL, FW>), grid, dim3(SL * FW * 64), 0, stream, p);
+    const dim3 grid(p.num_seqs, (p.pairs + 3) / 4, units * 4);
+    hipLaunchKernelGGL((merge_split_kernel<D, FW>), grid, dim3(FW * 64), 0, stream, p);
     return hipGetLastError();
 }
 
@@ -1884,10 +1925,13 @@ template <int D>
 hipError_t launch_merge_d(const DecodeParams& p, hipStream_t stream) {
     const int units = (min(8, p.group) * D + 255) / 256;  // per (sequence, kv-head slot)
     switch (merge_waves((int64_t)p.num_seqs * p.pairs * units)) {
-        case 8: return launch_merge_shape<D, 1, 8>(p, units, stream);
-        case 2: return launch_merge_shape<D, 1, 2>(p, units, stream);
-        default: return launch_merge_shape<D, (8 * D + 255) / 256, 1>(p, units, stream);
+        case 8: return launch_merge_shape<D, 8>(p, units, stream);
+        case 2: return launch_merge_shape<D, 2>(p, units, stream);
+        default: break;
     }
+    hipLaunchKernelGGL((merge_split_slot_kernel<D>), dim3(p.num_seqs, p.pairs), dim3((8 * D + 255) / 256 * 64), 0,
+                       stream, p);
+    return hipGetLastError();
 }
 
 hipError_t launch_merge_split(const DecodeParams& p, hipStream_t stream) {

@@ -21,31 +21,6 @@ __device__ __forceinline__ void remap_ids(const PrefillParams& p, int slots, int
     const int nx = gridDim.x, ny = gridDim.y;
     const int total = nx * ny * gridDim.z;
     const int C = p.xcd_cus;  // CUs per XCD
-    const int nz = gridDim.z;
-    // Grids of a few rounds (short prompts, uneven ones above all): an XCD
-    // serves nz / 8 of the z ids, the heaviest tiles of all its chunks first.
-    // Chunk by chunk, the last chunk's heavy tiles start when the others are
-    // done: six prompts of 9..700 tokens (32/8 heads of 128) 35.2 us against
-    // 29.5, on int8 pages 43.2 against 37.7, three of 300..1500 (16/16 of 64)
-    // 56.1 against 41.0.  The dispatcher goes round the CUs, so a period of
-    // (chunk, z) ids that divides them would leave a long chunk on a few CUs
-    // (8 chunks of 64..512 tokens, 32/8 of 128: 50.1 us; 39.2 with the chunks
-    // rotated by one per tile; 39.6 chunk by chunk).  In longer grids the
-    // balance matters less and the L2 more: 8 chunks of up to 2048 tokens on
-    // prefixes up to 4000 (int8) 720 us chunk by chunk, 801 like this.
-    // Key parts (splits) even the work out themselves: three ~40-token chunks on
-    // 7000-token prefixes 41.5 us chunk by chunk, 42.6 like this.
-    if (slots == 2 && C > 0 && p.splits <= 1 && nz % 8 == 0 && (total >> 3) <= 6 * C) {
-        const int lin = bx + nx * (by + ny * bz);
-        const int nzx = nz >> 3, per = total >> 3;
-        int j = lin >> 3;  // dispatch order within the XCD
-        if (per > C && per <= 2 * C && j >= C) j = per + C - 1 - j;  // one round: as below
-        const int q = j / nzx;
-        bz = (lin & 7) * nzx + j - q * nzx;
-        bx = q / ny;
-        by = C % (nzx * ny) == 0 ? (q + bx) % ny : q % ny;
-        return;
-    }
     if ((total & 7) == 0) {
         const int lin = bx + nx * (by + ny * bz);
         const int per = total >> 3;  // ids per XCD
@@ -74,17 +49,109 @@ __device__ __forceinline__ void remap_ids(const PrefillParams& p, int slots, int
     }
 }
 
-template <int KV, int D>
+// Small grids (prefill_live): workgroups placed by the chunks' real lengths,
+// which the host does not know, the heaviest tiles of all an XCD's chunks
+// first.  By the grid alone, chunk by chunk, the last chunk's heavy tiles
+// start when the others are done, and the workgroups of tiles that short
+// chunks do not have take turns on CUs: others then hold two live ones while
+// some hold none, however the grid is ordered (four chunks of 32..269 rows on
+// prefixes of 962..1378, 64/8 heads of 80: 46.7 us chunk by chunk, 62.3 with
+// the grid's heaviest tiles first, 46.9 by real lengths).
+// 5994 drawn calls against chunk by chunk: 0.972 of its time in the geometric
+// mean, 8 slower by over 5 % and none by over 6.1; by the grid's heaviest
+// tiles first 0.984, 24 slower by over 5 %, up to 34.  Six prompts of 9..700
+// tokens (32/8 heads of 128) 34.8 us chunk by chunk, 30.5 by the grid, 27.4.
+
+// The chunks' real lengths, one chunk per lane (at most 64): tiles of `rows`
+// query rows that the grid covers (the last ceil(max_chunk_len / rows) of a
+// longer chunk, a caller error), and their sum.
+struct LiveChunks {
+    int q0, n, prefix, tiles, total;
+    __device__ __forceinline__ LiveChunks(const PrefillParams& p, int rows, int lane) : q0(0), n(0), prefix(0) {
+        int end = 0;
+        if (lane < p.num_chunks) {
+            q0 = p.q_start[lane];
+            end = p.q_start[lane + 1];
+            prefix = p.prefix_lens[lane];
+        }
+        n = end - q0;
+        tiles = max(0, min((n + rows - 1) / rows, (p.max_chunk_len + rows - 1) / rows));
+        total = wave_sum(tiles);
+    }
+};
+
+// Place by weight (0: the heaviest) of the j-th of an XCD's `per` workgroups
+// on its C CUs.  The dispatcher gives each CU one before it gives any a second.
+__device__ __forceinline__ int live_rank(const LiveChunks& c, int j, int per, int C) {
+    if (per <= C || C <= 0) return j;
+    if (per <= 2 * C) {  // the heaviest alone, the lightest 2 (per - C) in pairs, heavy beside light
+        const int e = per - C;
+        return j < e ? C - e + j : j < C ? j - e : per + C - 1 - j;
+    }
+    // Up to a round and a half the heaviest tile's chain is the time: the
+    // second round lightest first, unless prefixes make the tiles alike.
+    if (per <= 3 * C && j >= C && j < 2 * C && wave_sum(c.tiles * ((2 * c.prefix - c.n) / 32)) < 0) return 3 * C - 1 - j;
+    return j;
+}
+
+// This workgroup's work by the chunks' real lengths; false: none.
+template <int QT>
+__device__ __forceinline__ bool live_work(const PrefillParams& p, PrefillWork& w) {
+    const int lane = threadIdx.x & 63;
+    const LiveChunks c(p, QT, lane);
+    const int nz = p.num_kv_heads * p.head_groups;
+    // grid (nz, tiles), an XCD's z ids nzx xcd .. + nzx - 1
+    const int xcd = blockIdx.x & 7, nzx = nz >> 3, per = c.total * nzx;
+    int q = blockIdx.y, zz = blockIdx.x >> 3;
+    const int j = zz + nzx * q;  // dispatch order within the XCD
+    if (j >= per) return false;
+    const int rank = live_rank(c, j, per, p.xcd_cus);
+    if (rank != j) {  // (a division that short calls need not wait for)
+        q = rank / nzx;
+        zz = rank - q * nzx;
+    }
+    // The q-th tile by its last key, in steps of a tile: level l holds at most
+    // one tile of a chunk, its (level - l)-th from the end.  (Levels are never
+    // below 0: the walk ends whatever the prefix lengths hold.)
+    const int level = max((c.prefix + c.n - 1) / QT, c.tiles - 1);
+    int l = wave_max0(c.tiles > 0 ? level : 0);
+    uint64_t m;
+    while (true) {
+        m = __ballot((uint32_t)(level - l) < (uint32_t)c.tiles);
+        const int cnt = __builtin_popcountll(m);
+        if (q < cnt) break;
+        q -= cnt;
+        l = cnt > 0 ? l - 1 : wave_max0(c.tiles > 0 && level < l ? level : 0);
+    }
+    const int at = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
+    const int by = __builtin_ctzll(__ballot((uint32_t)(level - l) < (uint32_t)c.tiles && at == q));
+    const int bx = __builtin_amdgcn_readlane(level, by) - l;
+    w = PrefillWork{bx, by, nzx * xcd + zz, 0, 1, __builtin_amdgcn_readlane(c.q0, by), __builtin_amdgcn_readlane(c.n, by),
+                    __builtin_amdgcn_readlane(c.prefix, by)};
+    return true;
+}
+
+template <int KV, int D, bool LIVE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void prefill_dma_kernel(PrefillParams p) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
-    int bx, by, bz;
-    remap_ids(p, 2, bx, by, bz);
-    // z: (key part, kv head, head group)
-    const int zh = p.num_kv_heads * p.head_groups;
-    const int part = bz / zh;
-    prefill_tile<KV, D, false>(p, bx, by, bz - part * zh, part,
-                               reinterpret_cast<lds_char*>((__attribute__((address_space(3))) char*)smem));
+    PrefillWork w;
+    if constexpr (LIVE) {
+        if (!live_work<16 * PDims<D>::RB>(p, w)) return;
+    } else {
+        int bx, by, bz;
+        remap_ids(p, 2, bx, by, bz);
+        // z: (key part, kv head, head group)
+        const int zh = p.num_kv_heads * p.head_groups;
+        w.bx = bx;
+        w.by = by;
+        w.part = bz / zh;
+        w.bz = bz - w.part * zh;
+        w.splits = p.splits;
+        w.load_chunk(p);
+    }
+    w.uniform();
+    prefill_tile<KV, D, false>(p, w, reinterpret_cast<lds_char*>((__attribute__((address_space(3))) char*)smem));
 }
 
 // fp16 pages at head_dim 64 / 80: 128-row tiles, one wave per SIMD
@@ -178,6 +245,43 @@ constexpr bool use_wide_t() { return KV == VCPP_KV_F16 && wide_prefill_ok<D>(); 
 
 bool pow2(int x) { return x > 0 && (x & (x - 1)) == 0; }
 
+// Whether a call of prefill_dma_kernel places its workgroups by the chunks'
+// real lengths (live_work): grids of up to three rounds of two workgroups per
+// CU, with more than one tile to a chunk and more than one chunk or head group
+// to an XCD.  In longer grids the balance matters less and the L2 more: 8
+// chunks of up to 2048 tokens on prefixes up to 4000 (int8) 720 us chunk by
+// chunk, 801 heaviest first.
+bool prefill_live(const PrefillParams& p) {
+    if (p.splits > 1 || p.num_chunks > 64 || prefill_uses_wide(p.kv_dtype, p.head_dim, p.block_size)) return false;
+    const int QT = prefill_tile_rows(p.kv_dtype, p.head_dim, p.block_size);
+    const int64_t nz = (int64_t)p.num_kv_heads * p.head_groups;
+    const int64_t total = (p.max_chunk_len + QT - 1) / QT * nz * p.num_chunks;
+    return (p.num_chunks > 1 || nz > 8) && p.max_chunk_len > QT && p.xcd_cus > 0 && nz % 8 == 0 && total <= 8 * 6 * p.xcd_cus;
+}
+
+// Raises a kernel's dynamic LDS limit on this device only when a launch needs
+// more than `set` last held there (the attribute call is a host round trip;
+// the limit is per device).
+hipError_t raise_lds(const void* fn, size_t (&set)[64], size_t lds) {
+    int dev = 0;
+    const bool known = hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < 64;
+    if (!known || lds > std::max<size_t>(set[dev], 65536)) {
+        const hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) return e;
+        if (known) set[dev] = lds;
+    }
+    return hipSuccess;
+}
+
+template <int KV, int D, bool LIVE>
+hipError_t launch_ring(const PrefillParams& p, dim3 grid, size_t lds, hipStream_t stream) {
+    static size_t attr_lds[64] = {};
+    const hipError_t e = raise_lds((const void*)prefill_dma_kernel<KV, D, LIVE>, attr_lds, lds);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL((prefill_dma_kernel<KV, D, LIVE>), grid, dim3(256), lds, stream, p);
+    return hipGetLastError();
+}
+
 template <int KV, int D>
 hipError_t launch_dma(const PrefillParams& p, hipStream_t stream) {
     const bool wide = prefill_uses_wide(KV, D, p.block_size);
@@ -189,33 +293,20 @@ hipError_t launch_dma(const PrefillParams& p, hipStream_t stream) {
 #ifdef VCPP_PREFILL_LDS_PAD
     lds = std::max<size_t>(lds, VCPP_PREFILL_LDS_PAD);
 #endif
-    // Raise the kernel's dynamic LDS limit on this device only when a launch
-    // needs more than it was last set to there (the attribute call is a host
-    // round trip; the limit is per device).
-    static size_t attr_lds[2][64] = {};
-    int dev = 0;
-    const bool known = hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < 64;
-    const void* fn = (const void*)prefill_dma_kernel<KV, D>;
-    if constexpr (use_wide_t<KV, D>()) {
-        if (wide) fn = (const void*)prefill_wide_kernel<D>;
-    }
-    if (!known || lds > std::max<size_t>(attr_lds[wide][dev], 65536)) {
-        const hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return e;
-        if (known) attr_lds[wide][dev] = lds;
-    }
+    const int64_t total = (int64_t)grid.x * grid.y * grid.z;
     if constexpr (use_wide_t<KV, D>()) {
         if (wide) {
             // A 1-D grid of all tiles (ordered by wide_tile_ids).
-            const unsigned tiles = grid.x * grid.y * grid.z;
-            hipLaunchKernelGGL((prefill_wide_kernel<D>), dim3(tiles), dim3(256), lds, stream, p);
+            static size_t attr_lds[64] = {};
+            const hipError_t e = raise_lds((const void*)prefill_wide_kernel<D>, attr_lds, lds);
+            if (e != hipSuccess) return e;
+            hipLaunchKernelGGL((prefill_wide_kernel<D>), dim3((unsigned)total), dim3(256), lds, stream, p);
             return hipGetLastError();
         }
     }
-    hipLaunchKernelGGL((prefill_dma_kernel<KV, D>), grid, dim3(256), lds, stream, p);
-    return hipGetLastError();
+    if (prefill_live(p)) return launch_ring<KV, D, true>(p, dim3(grid.z, grid.x * grid.y), lds, stream);
+    return launch_ring<KV, D, false>(p, grid, lds, stream);
 }
-
 
 }  // namespace
 

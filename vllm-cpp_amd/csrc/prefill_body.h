@@ -185,12 +185,33 @@ __device__ __forceinline__ float max_over_groups(float x) {
 }
 
 // One workgroup's work: query tile bx (0 = the chunk's last, heaviest tile)
-// of chunk by, kv head / head group bz, key part `part` of p.splits; lds is
-// the workgroup's dynamic LDS (prefill_lds_bytes).  Returns with every DMA it
-// issued complete.
+// of chunk by (rows q0 .. q0 + n - 1 after `prefix` positions), kv head / head
+// group bz, key part `part` of `splits`.
+struct PrefillWork {
+    int bx, by, bz, part, splits;
+    int q0, n, prefix;
+    __device__ __forceinline__ void load_chunk(const PrefillParams& p) {
+        q0 = p.q_start[by];
+        n = p.q_start[by + 1] - q0;
+        prefix = p.prefix_lens[by];
+    }
+    // The same values, provably wave-uniform (kept in SGPRs).
+    __device__ __forceinline__ void uniform() {
+        bx = __builtin_amdgcn_readfirstlane(bx);
+        by = __builtin_amdgcn_readfirstlane(by);
+        bz = __builtin_amdgcn_readfirstlane(bz);
+        part = __builtin_amdgcn_readfirstlane(part);
+        splits = __builtin_amdgcn_readfirstlane(splits);
+        q0 = __builtin_amdgcn_readfirstlane(q0);
+        n = __builtin_amdgcn_readfirstlane(n);
+        prefix = __builtin_amdgcn_readfirstlane(prefix);
+    }
+};
+
+// lds is the workgroup's dynamic LDS (prefill_lds_bytes).  Returns with every
+// DMA it issued complete.
 template <int KV, int D, bool F>
-__device__ __forceinline__ void prefill_tile(const PrefillParams& p, int bx, int by, int bz, int part,
-                                             lds_char* lds) {
+__device__ __forceinline__ void prefill_tile(const PrefillParams& p, const PrefillWork& w, lds_char* lds) {
     using DD = DmaDims<D, F>;
     constexpr bool BYTES = KV != VCPP_KV_F16;  // int8 / FP8: byte ring widened to fp16
     constexpr bool SCALED = KV == VCPP_KV_I8;  // per-key fp16 scales
@@ -212,13 +233,13 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int bx, int
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int g = lane >> 4, c = lane & 15;
-    const int chunk = by;
-    const int q0 = p.q_start[chunk], n = p.q_start[chunk + 1] - q0;
+    const int chunk = w.by, bz = w.bz, part = w.part, splits = w.splits;
+    const int q0 = w.q0, n = w.n;
     const int ntile = (n + kQTile - 1) / kQTile;
-    const int tile = ntile - 1 - bx;  // heaviest (latest) tiles first
+    const int tile = ntile - 1 - w.bx;  // heaviest (latest) tiles first
     if (tile < 0) return;             // whole workgroup: before any barrier
     const int t0 = tile * kQTile;
-    const int prefix = p.prefix_lens[chunk];
+    const int prefix = w.prefix;
     const int kvh = bz / p.head_groups;
     const int hg = bz - kvh * p.head_groups;
     const int hl = hg * kHeadsPerGroup + wave;
@@ -231,8 +252,8 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int bx, int
     // This part's key blocks [kb_lo, kb_hi): whole block pairs, the last part
     // up to nblk.
     const int npairs = (nblk + 1) / 2;
-    const int kb_lo = 2 * (int)((int64_t)part * npairs / p.splits);
-    const int kb_hi = min(2 * (int)((int64_t)(part + 1) * npairs / p.splits), nblk);
+    const int kb_lo = 2 * (int)((int64_t)part * npairs / splits);
+    const int kb_hi = min(2 * (int)((int64_t)(part + 1) * npairs / splits), nblk);
 
     // Q fragments (B operand of S^T = K Q^T).
     h8 qa[RB][NC32 > 0 ? NC32 : 1];
@@ -624,7 +645,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, int bx, int
     wait_vmcnt<0>();
 
     if (!head_ok) return;  // (no barrier follows)
-    if (p.splits > 1) {
+    if (splits > 1) {
         // Part outputs: o unnormalised, (m, l) of each row from lanes g == 0.
         const int64_t pbase = (int64_t)part * p.rows_cap;
 #pragma unroll

@@ -131,7 +131,7 @@ __device__ __forceinline__ bool live_work(const PrefillParams& p, PrefillWork& w
     return true;
 }
 
-template <int KV, int D, bool LIVE>
+template <int KV, int D, bool LIVE, int PB>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void prefill_dma_kernel(PrefillParams p) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -151,7 +151,7 @@ void prefill_dma_kernel(PrefillParams p) {
         w.load_chunk(p);
     }
     w.uniform();
-    prefill_tile<KV, D, false>(p, w, reinterpret_cast<lds_char*>((__attribute__((address_space(3))) char*)smem));
+    prefill_tile<KV, D, false, PB>(p, w, reinterpret_cast<lds_char*>((__attribute__((address_space(3))) char*)smem));
 }
 
 // fp16 pages at head_dim 64 / 80: 128-row tiles, one wave per SIMD
@@ -259,6 +259,17 @@ bool prefill_live(const PrefillParams& p) {
     return (p.num_chunks > 1 || nz > 8) && p.max_chunk_len > QT && p.xcd_cus > 0 && nz % 8 == 0 && total <= 8 * 6 * p.xcd_cus;
 }
 
+// Whether the four-stage fp16 ring (head_dim 128) takes two key blocks per
+// barrier after all: a grid of at most one workgroup per CU, over more than
+// 1024 keys to a part as far as the tables bound them.  A workgroup alone has
+// no other to cover its barriers: 35 rows on a prefix of 2800 (64/8 heads) 65.0
+// us in pairs, 67.8 one by one, 3 x 16 rows on 16000 341.5 against 363.7; but
+// 61 rows on 600 22.4 against 21.8.
+bool prefill_pairs(const PrefillParams& p, int64_t workgroups) {
+    return workgroups <= 8 * (int64_t)p.xcd_cus &&
+           (int64_t)p.max_blocks * p.block_size > 1024 * (int64_t)std::max(p.splits, 1);
+}
+
 // Raises a kernel's dynamic LDS limit on this device only when a launch needs
 // more than `set` last held there (the attribute call is a host round trip;
 // the limit is per device).
@@ -273,12 +284,12 @@ hipError_t raise_lds(const void* fn, size_t (&set)[64], size_t lds) {
     return hipSuccess;
 }
 
-template <int KV, int D, bool LIVE>
+template <int KV, int D, bool LIVE, int PB>
 hipError_t launch_ring(const PrefillParams& p, dim3 grid, size_t lds, hipStream_t stream) {
     static size_t attr_lds[64] = {};
-    const hipError_t e = raise_lds((const void*)prefill_dma_kernel<KV, D, LIVE>, attr_lds, lds);
+    const hipError_t e = raise_lds((const void*)prefill_dma_kernel<KV, D, LIVE, PB>, attr_lds, lds);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((prefill_dma_kernel<KV, D, LIVE>), grid, dim3(256), lds, stream, p);
+    hipLaunchKernelGGL((prefill_dma_kernel<KV, D, LIVE, PB>), grid, dim3(256), lds, stream, p);
     return hipGetLastError();
 }
 
@@ -304,8 +315,16 @@ hipError_t launch_dma(const PrefillParams& p, hipStream_t stream) {
             return hipGetLastError();
         }
     }
-    if (prefill_live(p)) return launch_ring<KV, D, true>(p, dim3(grid.z, grid.x * grid.y), lds, stream);
-    return launch_ring<KV, D, false>(p, grid, lds, stream);
+    constexpr int PB = DmaDims<D>::PER_BARRIER;
+    const bool live = prefill_live(p);
+    if (live) grid = dim3(grid.z, grid.x * grid.y);
+    if constexpr (KV == VCPP_KV_F16 && PB == 1) {
+        if (prefill_pairs(p, total))
+            return live ? launch_ring<KV, D, true, 2>(p, grid, lds, stream)
+                        : launch_ring<KV, D, false, 2>(p, grid, lds, stream);
+    }
+    return live ? launch_ring<KV, D, true, PB>(p, grid, lds, stream)
+                : launch_ring<KV, D, false, PB>(p, grid, lds, stream);
 }
 
 }  // namespace

@@ -111,7 +111,8 @@ struct DmaDims {
     // (D = 128: two workgroups' rings fill the LDS) take one, since pairs
     // would wait for the whole ring to drain before every pair: 8 chunks of
     // 2048 tokens on 1024-token prefixes, 32 heads of 128, 638 -> 615 us, one
-    // 512-token chunk on 16384, 167 -> 162 us.
+    // 512-token chunk on 16384, 167 -> 162 us.  (Workgroups alone on their CUs
+    // over long keys take pairs all the same: prefill_pairs.)
     static constexpr int PER_BARRIER = STAGES >= 6 || F ? 2 : 1;
     static_assert((2 * REGION) % 64 == 0, "stage must be whole DMA instructions");
 };
@@ -210,7 +211,7 @@ struct PrefillWork {
 
 // lds is the workgroup's dynamic LDS (prefill_lds_bytes).  Returns with every
 // DMA it issued complete.
-template <int KV, int D, bool F>
+template <int KV, int D, bool F, int PB = DmaDims<D, F>::PER_BARRIER>
 __device__ __forceinline__ void prefill_tile(const PrefillParams& p, const PrefillWork& w, lds_char* lds) {
     using DD = DmaDims<D, F>;
     constexpr bool BYTES = KV != VCPP_KV_F16;  // int8 / FP8: byte ring widened to fp16
@@ -617,8 +618,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillParams& p, const Prefi
             compute(kb, std::true_type{});
         }
     } else {
-        // Blocks consumed per barrier.
-        constexpr int PB = DD::PER_BARRIER;
+        // PB: blocks consumed per barrier.
 #pragma unroll
         for (int s = 0; s < kStages - PB; ++s) issue(kb_lo + s);
         auto step = [&](int kb) {

@@ -1,7 +1,9 @@
-"""The key parts vcpp_paged_prefill_split cuts a call into, read from what it
-says it needs where it is given no workspace: never more than fill two
-workgroups per CU, none that spills a few workgroups into a round of their
-own.  And the sizes vcpp_prefill_workspace_size gives for them."""
+"""The key parts vcpp_paged_prefill_split cuts a call into: the rule restated
+(prefill_split_cost and its callers), by the chunks' real lengths where a chunk
+can have several tiles (read back from a run's workspace in
+test_prefill_split_gpu.py), by the host's bounds otherwise (read from what a
+call says it needs where it is given no workspace).  And the sizes
+vcpp_prefill_workspace_size gives for them."""
 import ctypes
 import re
 
@@ -39,44 +41,67 @@ def need(chunks, rows, prefix, heads, kv_heads, dim):
     return int(re.search(r"needs (\d+) workspace bytes", pyvcpp.last_error()).group(1))
 
 
-def parts(chunks, rows, prefix, heads, kv_heads, dim):
-    got = need(chunks, rows, prefix, heads, kv_heads, dim)
-    for s in range(1, 17):
-        if got == bytes_of(s, chunks, rows, heads, dim):
-            return s
-    raise AssertionError("workspace of %d bytes is no whole number of parts" % got)
+def tile_rows(dim):
+    return 64 if dim <= 80 else 32
 
 
-# (chunks, rows, prefix, heads, kv heads, head_dim) on 256 CUs (what the
-# library assumes where there is no GPU to ask)
+def most_parts(chunks, rows, prefix, heads, kv_heads, dim, cus=256):
+    """prefill_most_splits."""
+    tiles = -(-rows // tile_rows(dim)) * chunks * kv_heads * -(-(heads // kv_heads) // 4)
+    return 1 if tiles >= 2 * cus else max(1, min(-(-2 * cus // tiles), (prefix + rows) // 512, 16))
+
+
+def parts(lens, prefixes, heads, kv_heads, dim, cus=256, caps=None):
+    """Parts of chunks of these lengths; caps: (max_chunk_len, max_prefix_len)."""
+    rows, prefix = caps or (max(lens), max(prefixes))
+    most = most_parts(len(lens), rows, prefix, heads, kv_heads, dim, cus)
+    if rows <= tile_rows(dim):  # the host's choice, by its bounds
+        lens, prefixes = [rows] * len(lens), [prefix] * len(lens)
+    zh = kv_heads * -(-(heads // kv_heads) // 4)
+    items = sum(-(-n // tile_rows(dim)) for n in lens) * zh
+    keys = max(n + p for n, p in zip(lens, prefixes) if n > 0)
+
+    def cost(s):
+        full, rest = divmod(items * s, 2 * cus)
+        return (keys / (32 * s) * (full + (0 if rest == 0 else 0.72 if rest <= cus else 1)) + 5 * (full + (rest > 0)) +
+                (s * sum(lens) * heads * dim * 8 / 6.5e6 if s > 1 else 0))
+
+    live = rows > tile_rows(dim)
+    return min((s for s in range(1, most + 1) if s == 1 or not live or s * 512 <= keys), key=cost)
+
+
+# (row counts, prefixes, heads, kv heads, head_dim)
 @pytest.mark.parametrize("call,want", [
-    ((3, 50, 7000, 32, 8, 128), 10),     # 48 tiles: 11 parts would be 528 workgroups
-    ((1, 512, 32768, 64, 8, 80), 4),     # 128 tiles: two per CU exactly
-    ((1, 300, 16384, 64, 8, 80), 6),     # 80 tiles
-    ((3, 500, 8192, 64, 8, 80), 2),      # 384 tiles: a round and a half of halves beats one of wholes
-    ((8, 2048, 1024, 64, 8, 80), 1),     # the chunks fill the GPU
-    ((1, 16, 400, 8, 8, 64), 1),         # too short to cut
-    ((1, 16, 100000, 8, 1, 64), 16)])
+    (([50, 50, 50], [7000] * 3, 32, 8, 128), 10),     # 48 tiles: 11 parts would be 528 workgroups
+    (([512], [32768], 64, 8, 80), 4),                 # 128 tiles: two per CU exactly
+    (([300], [16384], 64, 8, 80), 6),                 # 80 tiles
+    (([500] * 3, [8192] * 3, 64, 8, 80), 2),          # 384 tiles: a round and a half of halves beats one of wholes
+    (([449, 387, 178], [18453, 19757, 14792], 24, 8, 80), 3),  # 144 real tiles of the grid's 192, which take two
+    (([244, 357], [17221, 15921], 64, 8, 64), 3),
+    (([2048] * 8, [1024] * 8, 64, 8, 80), 1),         # the chunks fill the GPU
+    (([16], [400], 8, 8, 64), 1),                     # too short to cut
+    (([16], [100000], 8, 1, 64), 16)])
 def test_parts(call, want):
     assert parts(*call) == want
 
 
-def test_parts_bound():
-    """Never more parts than fill two workgroups per CU, so the workspace is
-    within what that count needs; whole tiles only."""
-    for chunks in (1, 2, 5):
-        for rows in (1, 33, 64, 200, 511):
+def test_one_tile_a_chunk():
+    """The host's choice where a chunk has one tile at most: never more than
+    the fullest count, and the restated rule's."""
+    for chunks in (1, 2, 5, 20):
+        for rows in (1, 31, 32, 33, 64):
             for prefix in (0, 700, 5000, 40000):
                 for heads, kv_heads, dim in ((64, 8, 80), (28, 4, 128), (8, 8, 64)):
-                    tiles = -(-rows // (64 if dim <= 80 else 32)) * chunks * kv_heads * -(-(heads // kv_heads) // 4)
-                    most = max(1, min(-(-512 // tiles), (prefix + rows) // 512, 16))
-                    assert 1 <= parts(chunks, rows, prefix, heads, kv_heads, dim) <= most
+                    if rows > tile_rows(dim):
+                        continue
+                    s = parts([rows] * chunks, [prefix] * chunks, heads, kv_heads, dim)
+                    assert need(chunks, rows, prefix, heads, kv_heads, dim) == bytes_of(s, chunks, rows, heads, dim)
 
 
 def test_size_at_caps_covers_smaller_calls():
-    """A buffer sized once for an engine's limits: 512 rows and 320 rows of
-    three chunks (one part and two), and the size of every call is that of
-    the fullest split, whose rows times parts do not jump with the rows."""
+    """A buffer sized once for an engine's limits, 512 rows of three chunks,
+    holds shorter calls' partials; the size of every call is that of the
+    fullest split, whose rows times parts do not jump with the rows."""
     cap = size(3, 512, 2000, 64, 8, 64)
     for rows in range(8, 513, 8):
         assert need(3, rows, 2000, 64, 8, 64) <= cap, rows
@@ -84,9 +109,7 @@ def test_size_at_caps_covers_smaller_calls():
         for rows in (1, 33, 64, 200, 320, 511, 512):
             for prefix in (0, 700, 2000, 5000, 40000):
                 for heads, kv_heads, dim in ((64, 8, 80), (28, 4, 128), (8, 8, 64), (64, 8, 64)):
-                    tiles = -(-rows // (64 if dim <= 80 else 32)) * chunks * kv_heads * -(-(heads // kv_heads) // 4)
-                    most = 1 if tiles >= 512 else max(1, min(-(-512 // tiles), (prefix + rows) // 512, 16))
                     call = (chunks, rows, prefix, heads, kv_heads, dim)
-                    assert size(*call) == bytes_of(most, chunks, rows, heads, dim), call
+                    assert size(*call) == bytes_of(most_parts(*call), chunks, rows, heads, dim), call
                     assert need(*call) <= size(*call), call
                     assert size(*call) <= 1024 * 256 * (4 * dim + 8) // (2 if dim == 128 else 1) + 256, call

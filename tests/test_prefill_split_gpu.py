@@ -136,3 +136,38 @@ def test_chunk_longer_than_max_chunk_len(cuda, split):
     if not split:  # (the split path stores only rows below num_chunks * max_chunk_len = 128)
         assert not rows_nan[192:200].any(), "the chunk's last tile was not computed"
     assert_close(got[~rows_nan], want[~rows_nan], ATOL, RTOL, what="written rows, split=%s" % split)
+
+
+@pytest.mark.parametrize("lens,prefixes,H,Hkv,D,caps", [
+    ([70, 40], [3000, 2100], 64, 8, 128, None),         # 5 of the grid's 6 tiles a head group
+    ([130, 3, 65], [1900, 2500, 600], 16, 16, 64, None),
+    ([130, 3, 65], [1900, 2500, 600], 16, 16, 64, (200, 6000)),  # the caller's bounds loose: parts by the real keys
+    ([33, 0, 1], [1000, 0, 5], 8, 1, 128, None),        # an empty chunk
+    ([90], [200], 64, 8, 80, (90, 9000)),               # the real keys are too few to cut: finished in place
+    ([20, 9, 31], [3000, 800, 1700], 32, 8, 128, None), # one tile a chunk: the host's count
+    ([33] * 65, [1100] * 65, 1, 1, 128, None)])          # more chunks than lanes: the fullest count
+def test_parts_by_real_lengths(cuda, lens, prefixes, H, Hkv, D, caps):
+    """The count the workgroups and the merge choose by the device's lengths is
+    the restated rule's: parts past it leave their workspace as it was."""
+    from test_prefill_parts import most_parts, parts
+    rows, prefix = caps or (max(lens), max(prefixes))
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    most = most_parts(len(lens), rows, prefix, H, Hkv, D, cus)
+    host = parts(lens, prefixes, H, Hkv, D, cus, caps)
+    want_parts = most if len(lens) > 64 else host
+    assert most > 1
+    pool, q16, q32, tables, q_start, pre = make_case(O.ORC_F16, 760 + D, prefixes, lens, H, Hkv, D)
+    want = O.prefill(pool, q32, tables, q_start, pre, H)
+    dp = DevPool(pool)
+    q, out = dev(q16), torch.full((int(q_start[-1]), H, D), float("nan"), device="cuda:0")
+    need = pyvcpp.prefill_workspace_size(dp.pages, len(lens), rows, prefix, H)
+    ws = torch.full((need // 4,), float("nan"), device="cuda:0")
+    pyvcpp.paged_prefill_split(dp.pages, q, out, dev(tables), dev(q_start), dev(pre), rows, prefix, H,
+                               workspace=ws.view(torch.uint8))
+    torch.cuda.synchronize()
+    assert_close(out.cpu().numpy(), want, ATOL, RTOL, what="split parts %s" % (lens,))
+    if rows <= 32:
+        return  # (test_prefill_parts.py)
+    slab = len(lens) * rows * H * D  # of one part's outputs, first row of the first chunk in its head
+    written = [s for s in range(most) if not torch.isnan(ws[s * slab])]
+    assert written == (list(range(want_parts)) if want_parts > 1 else [])

@@ -639,9 +639,7 @@ static int64_t prefill_items(const vcpp_kv_pages* kv, int32_t num_chunks, int32_
 // sized for: enough workgroups to fill two per CU, each part at least 16 key
 // blocks (512 keys) of the longest chunk, at most 16.  The rows times parts of
 // this count change little with the call's rows, so that a buffer sized for a
-// longer call mostly holds a shorter one's partials; those of prefill_splits'
-// own count jump (three chunks on 2000-token prefixes, 64/8 heads of 64: one
-// part at 512 rows, two at 320).
+// longer call mostly holds a shorter one's partials.
 static int32_t prefill_most_splits(const vcpp_kv_pages* kv, int32_t num_chunks, int32_t max_chunk_len,
                                    int32_t max_prefix_len, int32_t num_heads) {
     if (num_chunks <= 0 || max_chunk_len <= 0 || max_prefix_len < 0) return 1;
@@ -653,36 +651,27 @@ static int32_t prefill_most_splits(const vcpp_kv_pages* kv, int32_t num_chunks, 
     return (int32_t)std::max<int64_t>(1, std::min<int64_t>({want, by_len, (int64_t)vcpp::kMaxPrefillSplits}));
 }
 
-// Key parts of a split prefill: of 1 .. prefill_most_splits the count that a
-// sum of the launch's rounds puts first.  In units of one 32-key block of two
-// resident workgroups per CU (about 1.3 us): a round of a part's blocks, 0.65
-// of that where the last round leaves one workgroup per CU, 5 for a round's
-// start and end, and the partials' traffic.  The fullest count is not it where
-// it spills a few workgroups into a round of their own: 48 tiles in 11 parts
-// are 528 workgroups, 56.0 us for three 40-token chunks on 7000-token prefixes
-// (32/8 heads of 128), 41.9 in 10 parts; one 300-token chunk on 16384, 146.9
-// in 7 parts, 111.8 in 6.  But 384 tiles (three 500-token chunks on 8192, 64/8
-// heads of 80) take 365 us whole and 325 in two parts.
-static int32_t prefill_splits(const vcpp_kv_pages* kv, int32_t num_chunks, int32_t max_chunk_len,
-                              int32_t max_prefix_len, int32_t num_heads) {
-    const int32_t most = prefill_most_splits(kv, num_chunks, max_chunk_len, max_prefix_len, num_heads);
-    if (most == 1) return 1;
-    const int64_t items = prefill_items(kv, num_chunks, max_chunk_len, num_heads);
-    const int64_t cus = device_cus(), slots = 2 * cus;
-    const double blocks = ((double)max_prefix_len + max_chunk_len) / 32;
-    const double part_bytes = 8.0 * num_chunks * max_chunk_len * num_heads * kv->head_dim;  // written and read
-    int32_t best = 1;
-    double best_cost = 0;
-    for (int32_t s = 1; s <= most; ++s) {
-        const int64_t full = items * s / slots, rest = items * s % slots;
-        const double cost = blocks / s * (full + (rest == 0 ? 0.0 : rest <= cus ? 0.65 : 1.0)) +
-                            5.0 * (full + (rest > 0)) + (s > 1 ? s * part_bytes / 6.5e6 : 0.0);
-        if (s == 1 || cost < best_cost) {
-            best = s;
-            best_cost = cost;
-        }
+// Key parts of a split call: where a chunk can have several tiles, up to
+// prefill_most_splits by the lengths the device holds (`live`, the workgroups'
+// choice); with one tile to a chunk the count of least cost, chosen here.  More
+// than 64 chunks (and the wide kernel): the fullest count.
+static void choose_splits(vcpp::PrefillParams& p, const vcpp_kv_pages* kv, int32_t max_prefix_len) {
+    p.splits = prefill_most_splits(kv, p.num_chunks, p.max_chunk_len, max_prefix_len, p.num_heads);
+    if (p.splits == 1 || p.num_chunks > 64 || vcpp::prefill_uses_wide(kv->dtype, kv->head_dim, kv->block_size)) return;
+    if (p.max_chunk_len > vcpp::prefill_tile_rows(kv->dtype, kv->head_dim, kv->block_size)) {
+        p.live = 1;
+        return;
     }
-    return best;
+    const int32_t items = (int32_t)prefill_items(kv, p.num_chunks, p.max_chunk_len, p.num_heads), cus = device_cus();
+    const float keys = (float)max_prefix_len + p.max_chunk_len;
+    const float out_values = (float)p.num_chunks * p.max_chunk_len * p.num_heads * kv->head_dim;
+    const auto cost = [&](int32_t s) {
+        return vcpp::prefill_split_cost(s, items, items * s / (2 * cus), keys, out_values, cus);
+    };
+    int32_t best = 1;
+    for (int32_t s = 2; s <= p.splits; ++s)
+        if (cost(s) < cost(best)) best = s;
+    p.splits = best;
 }
 
 size_t vcpp_prefill_workspace_size(const vcpp_kv_pages* kv, int32_t num_chunks, int32_t max_chunk_len,
@@ -705,7 +694,7 @@ int vcpp_paged_prefill_split(const vcpp_kv_pages* kv, const uint16_t* q, float* 
     if (max_prefix_len < 0) return fail(VCPP_E_INVALID, "max_prefix_len must be >= 0");
     vcpp::PrefillParams p = prefill_params(kv, q, out, block_tables, max_blocks_per_seq, q_start, prefix_lens,
                                            num_chunks, max_chunk_len, num_heads);
-    p.splits = prefill_splits(kv, num_chunks, max_chunk_len, max_prefix_len, num_heads);
+    choose_splits(p, kv, max_prefix_len);
     if ((int64_t)kv->num_kv_heads * p.head_groups * p.splits > 65535)
         return fail(VCPP_E_UNSUPPORTED, "too many heads x key parts");
     if (p.splits > 1) {

@@ -39,6 +39,7 @@ struct PrefillParams {
     // unnormalised outputs and (max, sum) in ws_o / ws_ml at row
     // k * rows_cap + row, for launch_prefill's merge
     int32_t splits;
+    int32_t live;      // 1: in 1 .. splits parts, by the chunks' real lengths (live_splits)
     int32_t rows_cap;  // >= the rows of all chunks (num_chunks * max_chunk_len)
     float* ws_o;       // [splits][rows_cap][num_heads][head_dim]
     float2* ws_ml;     // [splits][rows_cap][num_heads] (max in log2 units, sum)
@@ -50,6 +51,24 @@ struct PrefillParams {
     int64_t gather_stride;
 #endif
 };
+
+// Cost of a split call in s key parts, of `items` workgroups a part whose
+// longest keys are `keys`, in units of one 32-key block of two resident
+// workgroups per CU (about 1.3 us): a round of a part's blocks, 0.72 of that
+// where the last round leaves one workgroup per CU, 5 for a round's start and
+// end, and the partials' traffic.  The fullest count is not the best where it
+// spills a few workgroups into a round of their own: 48 tiles in 11 parts are
+// 528 workgroups, 56.0 us for three 40-token chunks on 7000-token prefixes
+// (32/8 heads of 128), 41.9 in 10 parts; but 384 tiles (three 500-token chunks
+// on 8192, 64/8 heads of 80) take 365 us whole and 325 in two parts.  Over 3746
+// drawn calls, each timed at every count, the count of least cost takes 1.0015
+// of the best one's time in the geometric mean, 0.952 of the fullest one's.
+// (full: items * s / (2 * cus), whole rounds.)
+__host__ __device__ inline float prefill_split_cost(int s, int items, int full, float keys, float out_values, int cus) {
+    const int rest = items * s - full * 2 * cus;
+    return keys / (32.f * s) * (full + (rest == 0 ? 0.f : rest <= cus ? 0.72f : 1.f)) + 5.f * (full + (rest > 0)) +
+           (s > 1 ? s * out_values * (8.f / 6.5e6f) : 0.f);
+}
 
 hipError_t launch_prefill(const PrefillParams& p, hipStream_t stream);
 // Workspace bytes of a split prefill (0 when splits <= 1).

@@ -66,7 +66,7 @@ __device__ __forceinline__ void remap_ids(const PrefillParams& p, int slots, int
 // query rows that the grid covers (the last ceil(max_chunk_len / rows) of a
 // longer chunk, a caller error), and their sum.
 struct LiveChunks {
-    int q0, n, prefix, tiles, total;
+    int q0, n, prefix, tiles, incl, total;
     __device__ __forceinline__ LiveChunks(const PrefillParams& p, int rows, int lane) : q0(0), n(0), prefix(0) {
         int end = 0;
         if (lane < p.num_chunks) {
@@ -76,7 +76,8 @@ struct LiveChunks {
         }
         n = end - q0;
         tiles = max(0, min((n + rows - 1) / rows, (p.max_chunk_len + rows - 1) / rows));
-        total = wave_sum(tiles);
+        incl = wave_incl_scan(tiles);
+        total = __builtin_amdgcn_readlane(incl, 63);
     }
 };
 
@@ -131,13 +132,82 @@ __device__ __forceinline__ bool live_work(const PrefillParams& p, PrefillWork& w
     return true;
 }
 
-template <int KV, int D, bool LIVE, int PB>
+// a / b for 0 <= a < 2^22, b > 0: a reciprocal and one correction, a third of
+// the integer division's chain.
+__device__ __forceinline__ int div_small(int a, int b) {
+    int q = (int)((float)a * __builtin_amdgcn_rcpf((float)b));
+    const int r = a - q * b;
+    q += r >= b ? 1 : r < 0 ? -1 : 0;
+    return q;
+}
+
+// Key parts of a split call by the chunks' real lengths: of 1 .. p.splits the
+// count of least cost, at least 512 keys of the longest chunk to a part.  By
+// max_chunk_len the host would count tiles that short chunks do not have, and
+// so take too few parts (three chunks of 178..449 rows on prefixes up to 19757,
+// 24/8 heads of 80: 432 us in two parts, 301 in three).  Lane s - 1 weighs s
+// parts, and every workgroup and the merge come to the same count.
+__device__ __forceinline__ int live_splits(const PrefillParams& p, const LiveChunks& c, int lane) {
+    const int keys = wave_max0(c.tiles > 0 ? c.prefix + c.n : 0);
+    const int last = p.num_chunks - 1;
+    const int rows = __builtin_amdgcn_readlane(c.q0 + c.n, last) - __builtin_amdgcn_readlane(c.q0, 0);
+    const float out_values = (float)rows * (p.num_heads * p.head_dim);
+    const int items = c.total * p.num_kv_heads * p.head_groups, cus = max(8 * p.xcd_cus, 1);
+    const int s = lane + 1;
+    uint32_t best = ~0u;  // cost (positive: its bits are ordered), low bits the count
+    if (s <= p.splits && (s == 1 || s * 512 <= keys)) {
+        const float cost = prefill_split_cost(s, items, div_small(items * s, 2 * cus), (float)keys, out_values, cus);
+        best = ((uint32_t)__float_as_int(cost) & ~15u) | lane;
+    }
+    static_assert(kMaxPrefillSplits == 16, "counts in four bits, of one row of lanes");
+    // (rotations of the row; a shuffle's lane addresses would stay in registers)
+    best = min(best, (uint32_t)__builtin_amdgcn_mov_dpp((int)best, 0x128, 0xF, 0xF, false));
+    best = min(best, (uint32_t)__builtin_amdgcn_mov_dpp((int)best, 0x124, 0xF, 0xF, false));
+    best = min(best, (uint32_t)__builtin_amdgcn_mov_dpp((int)best, 0x122, 0xF, 0xF, false));
+    best = min(best, (uint32_t)__builtin_amdgcn_mov_dpp((int)best, 0x121, 0xF, 0xF, false));
+    return (__builtin_amdgcn_readlane((int)best, 0) & 15) + 1;
+}
+
+// This workgroup's work of a split call, in `splits` parts; false: none.
+template <int QT>
+__device__ __forceinline__ bool live_split_work(const PrefillParams& p, PrefillWork& w) {
+    const int lane = threadIdx.x & 63;
+    const LiveChunks c(p, QT, lane);
+    const int splits = live_splits(p, c, lane);
+    const int C = p.xcd_cus, HG = p.head_groups;
+    const int one = c.total * HG, total = one * p.num_kv_heads * splits, per = (total + 7) >> 3;
+    int j = blockIdx.x >> 3;  // dispatch order within the XCD
+    if (j >= per) return false;
+    if (per > C && per <= 2 * C && j >= C) j = per + C - 1 - j;  // one round: as in remap_ids
+    const int m = (int)(blockIdx.x & 7) * per + j;
+    if (m >= total) return false;
+    // m = tile + tiles (head group + HG (chunks before + ..)), then kv head, part
+    const int y = __builtin_amdgcn_readfirstlane(div_small(m, one)), r = m - y * one;
+    const int part = __builtin_amdgcn_readfirstlane(div_small(y, p.num_kv_heads));
+    const int excl = c.incl - c.tiles;
+    const int by = __builtin_popcountll(__ballot(lane < p.num_chunks && excl * HG <= r)) - 1;
+    const int rr = r - HG * __builtin_amdgcn_readlane(excl, by);
+    const int nt = __builtin_amdgcn_readlane(c.tiles, by);
+    const int hg = __builtin_amdgcn_readfirstlane(div_small(rr, nt));
+    w = PrefillWork{rr - hg * nt, by, (y - part * p.num_kv_heads) * HG + hg, part, splits,
+                    __builtin_amdgcn_readlane(c.q0, by), __builtin_amdgcn_readlane(c.n, by),
+                    __builtin_amdgcn_readlane(c.prefix, by)};
+    return true;
+}
+
+// PLACE: by the grid (remap_ids), or by the chunks' real lengths, unsplit
+// (live_work) or split (live_split_work).
+enum { kGrid = 0, kLive = 1, kLiveSplit = 2 };
+
+template <int KV, int D, int PLACE, int PB>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void prefill_dma_kernel(PrefillParams p) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     PrefillWork w;
-    if constexpr (LIVE) {
+    if constexpr (PLACE == kLive) {
         if (!live_work<16 * PDims<D>::RB>(p, w)) return;
+    } else if constexpr (PLACE == kLiveSplit) {
+        if (!live_split_work<16 * PDims<D>::RB>(p, w)) return;
     } else {
         int bx, by, bz;
         remap_ids(p, 2, bx, by, bz);
@@ -170,6 +240,15 @@ template <int S>
 __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillParams p) {
     const int D4 = p.head_dim / 4;
     const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    int parts = S;
+    bool too_long = true;  // chunks longer than max_chunk_len to look for
+    if (p.live) {
+        const int lane = threadIdx.x & 63;
+        const LiveChunks c(p, p.tile_rows, lane);
+        parts = live_splits(p, c, lane);
+        if (parts <= 1) return;  // finished in place
+        too_long = __any(c.n > c.tiles * p.tile_rows);
+    }
     const int64_t per_row = (int64_t)p.num_heads * D4;
     const int row = (int)(idx / per_row);
     if (row >= p.q_start[p.num_chunks]) return;
@@ -177,7 +256,7 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillParams p) {
     // query tile of the grid covered are left unwritten, as the unsplit
     // kernel leaves them: the grid covers each chunk's last
     // ceil(max_chunk_len / tile_rows) tiles.
-    {
+    if (too_long) {
         int lo = 0, hi = p.num_chunks - 1;  // chunk of the row: last c with q_start[c] <= row
         while (lo < hi) {
             const int mid = (lo + hi + 1) >> 1;
@@ -196,8 +275,10 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillParams p) {
     float M = -__builtin_inff();
 #pragma unroll
     for (int s = 0; s < S; ++s) {
-        const int64_t rh = ((int64_t)s * p.rows_cap + row) * p.num_heads + head;
+        // (parts past the count are not there: part 0 again, with weight 0)
+        const int64_t rh = ((int64_t)(s < parts ? s : 0) * p.rows_cap + row) * p.num_heads + head;
         ml[s] = p.ws_ml[rh];
+        if (s >= parts) ml[s].y = 0.f;
         v[s] = reinterpret_cast<const float4*>(p.ws_o + rh * p.head_dim)[d4];
     }
 #pragma unroll
@@ -284,12 +365,12 @@ hipError_t raise_lds(const void* fn, size_t (&set)[64], size_t lds) {
     return hipSuccess;
 }
 
-template <int KV, int D, bool LIVE, int PB>
+template <int KV, int D, int PLACE, int PB>
 hipError_t launch_ring(const PrefillParams& p, dim3 grid, size_t lds, hipStream_t stream) {
     static size_t attr_lds[64] = {};
-    const hipError_t e = raise_lds((const void*)prefill_dma_kernel<KV, D, LIVE, PB>, attr_lds, lds);
+    const hipError_t e = raise_lds((const void*)prefill_dma_kernel<KV, D, PLACE, PB>, attr_lds, lds);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((prefill_dma_kernel<KV, D, LIVE, PB>), grid, dim3(256), lds, stream, p);
+    hipLaunchKernelGGL((prefill_dma_kernel<KV, D, PLACE, PB>), grid, dim3(256), lds, stream, p);
     return hipGetLastError();
 }
 
@@ -316,15 +397,16 @@ hipError_t launch_dma(const PrefillParams& p, hipStream_t stream) {
         }
     }
     constexpr int PB = DmaDims<D>::PER_BARRIER;
+    if (p.live) return launch_ring<KV, D, kLiveSplit, PB>(p, dim3((unsigned)((total + 7) / 8 * 8)), lds, stream);
     const bool live = prefill_live(p);
     if (live) grid = dim3(grid.z, grid.x * grid.y);
     if constexpr (KV == VCPP_KV_F16 && PB == 1) {
         if (prefill_pairs(p, total))
-            return live ? launch_ring<KV, D, true, 2>(p, grid, lds, stream)
-                        : launch_ring<KV, D, false, 2>(p, grid, lds, stream);
+            return live ? launch_ring<KV, D, kLive, 2>(p, grid, lds, stream)
+                        : launch_ring<KV, D, kGrid, 2>(p, grid, lds, stream);
     }
-    return live ? launch_ring<KV, D, true, PB>(p, grid, lds, stream)
-                : launch_ring<KV, D, false, PB>(p, grid, lds, stream);
+    return live ? launch_ring<KV, D, kLive, PB>(p, grid, lds, stream)
+                : launch_ring<KV, D, kGrid, PB>(p, grid, lds, stream);
 }
 
 }  // namespace

@@ -55,7 +55,10 @@ def parts(lens, prefixes, heads, kv_heads, dim, cus=256, caps=None):
     """Parts of chunks of these lengths; caps: (max_chunk_len, max_prefix_len)."""
     rows, prefix = caps or (max(lens), max(prefixes))
     most = most_parts(len(lens), rows, prefix, heads, kv_heads, dim, cus)
-    if rows <= tile_rows(dim):  # the host's choice, by its bounds
+    live = rows > tile_rows(dim)
+    if live and len(lens) == 1 and caps and parts([rows], [prefix], heads, kv_heads, dim, cus) == most:
+        return most  # one chunk's fullest count, by the host's bounds
+    if not live:
         lens, prefixes = [rows] * len(lens), [prefix] * len(lens)
     zh = kv_heads * -(-(heads // kv_heads) // 4)
     items = sum(-(-n // tile_rows(dim)) for n in lens) * zh
@@ -66,7 +69,6 @@ def parts(lens, prefixes, heads, kv_heads, dim, cus=256, caps=None):
         return (keys / (32 * s) * (full + (0 if rest == 0 else 0.72 if rest <= cus else 1)) + 5 * (full + (rest > 0)) +
                 (s * sum(lens) * heads * dim * 8 / 6.5e6 if s > 1 else 0))
 
-    live = rows > tile_rows(dim)
     return min((s for s in range(1, most + 1) if s == 1 or not live or s * 512 <= keys), key=cost)
 
 
@@ -83,6 +85,14 @@ def parts(lens, prefixes, heads, kv_heads, dim, cus=256, caps=None):
     (([16], [100000], 8, 1, 64), 16)])
 def test_parts(call, want):
     assert parts(*call) == want
+
+
+def test_one_chunk_loose_bounds():
+    """A single chunk far shorter than its bound: the fullest count where that
+    is the bound's best one, by the real lengths where it is not."""
+    assert parts([100], [30000], 64, 8, 80, caps=(512, 32768)) == 4
+    assert parts([100], [16000], 64, 8, 80, caps=(300, 16384)) == 7  # 6 by the bounds
+    assert parts([90], [200], 64, 8, 80, caps=(300, 16384)) == 1
 
 
 def test_one_tile_a_chunk():

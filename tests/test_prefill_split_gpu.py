@@ -143,7 +143,8 @@ def test_chunk_longer_than_max_chunk_len(cuda, split):
     ([130, 3, 65], [1900, 2500, 600], 16, 16, 64, None),
     ([130, 3, 65], [1900, 2500, 600], 16, 16, 64, (200, 6000)),  # the caller's bounds loose: parts by the real keys
     ([33, 0, 1], [1000, 0, 5], 8, 1, 128, None),        # an empty chunk
-    ([90], [200], 64, 8, 80, (90, 9000)),               # the real keys are too few to cut: finished in place
+    ([90], [200], 64, 8, 80, (300, 9000)),              # the real keys are too few to cut: finished in place
+    ([90], [200], 64, 8, 80, (90, 9000)),               # one chunk's fullest count, more parts than key blocks
     ([20, 9, 31], [3000, 800, 1700], 32, 8, 128, None), # one tile a chunk: the host's count
     ([33] * 65, [1100] * 65, 1, 1, 128, None)])          # more chunks than lanes: the fullest count
 def test_parts_by_real_lengths(cuda, lens, prefixes, H, Hkv, D, caps):

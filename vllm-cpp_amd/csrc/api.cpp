@@ -122,6 +122,11 @@ struct DecodePlan {
 // where 64-token partitions would be too many (16 x 512, 14.0 against 14.5).
 // More than 128 partitions cost the merge more than the shorter ones save (1 x
 // 32768 with 12/2 heads of 128: 18.6 us at 128 tokens, 15.0 at 256).
+// max_ctx is the caller's bound, so real lengths far below it leave workgroups
+// without tokens.  Bounds of 4 and 16 times the lengths, and one long sequence
+// among short ones (108 such calls), are still 1.0 to 4 times as fast as the
+// general path, but for 8 sequences of about 2000 tokens bounded at 32768 (12/2
+// heads of 128, byte pages): 27.2 us against 24.5.
 int32_t small_partition(int64_t units, int32_t max_ctx, bool page_mode) {
     const int64_t most = std::min<int64_t>(2 * device_cus(), 1000);  // (decode.hip's kSeqsShift)
     if (units > most) return 0;
@@ -651,17 +656,14 @@ static int32_t prefill_most_splits(const vcpp_kv_pages* kv, int32_t num_chunks, 
     return (int32_t)std::max<int64_t>(1, std::min<int64_t>({want, by_len, (int64_t)vcpp::kMaxPrefillSplits}));
 }
 
-// Key parts of a split call: where a chunk can have several tiles, up to
-// prefill_most_splits by the lengths the device holds (`live`, the workgroups'
-// choice); with one tile to a chunk the count of least cost, chosen here.  More
-// than 64 chunks (and the wide kernel): the fullest count.
+// Key parts of a split call.  The count of least cost by the host's bounds is
+// the call's where they say it all (one tile to a chunk) or where it is one
+// chunk's fullest count anyway; otherwise up to prefill_most_splits by the
+// lengths the device holds (`live`, the workgroups' choice, about 1.5 us of a
+// 380 us call).  More than 64 chunks (and the wide kernel): the fullest count.
 static void choose_splits(vcpp::PrefillParams& p, const vcpp_kv_pages* kv, int32_t max_prefix_len) {
     p.splits = prefill_most_splits(kv, p.num_chunks, p.max_chunk_len, max_prefix_len, p.num_heads);
     if (p.splits == 1 || p.num_chunks > 64 || vcpp::prefill_uses_wide(kv->dtype, kv->head_dim, kv->block_size)) return;
-    if (p.max_chunk_len > vcpp::prefill_tile_rows(kv->dtype, kv->head_dim, kv->block_size)) {
-        p.live = 1;
-        return;
-    }
     const int32_t items = (int32_t)prefill_items(kv, p.num_chunks, p.max_chunk_len, p.num_heads), cus = device_cus();
     const float keys = (float)max_prefix_len + p.max_chunk_len;
     const float out_values = (float)p.num_chunks * p.max_chunk_len * p.num_heads * kv->head_dim;
@@ -671,7 +673,9 @@ static void choose_splits(vcpp::PrefillParams& p, const vcpp_kv_pages* kv, int32
     int32_t best = 1;
     for (int32_t s = 2; s <= p.splits; ++s)
         if (cost(s) < cost(best)) best = s;
-    p.splits = best;
+    const bool several = p.max_chunk_len > vcpp::prefill_tile_rows(kv->dtype, kv->head_dim, kv->block_size);
+    if (several && (p.num_chunks > 1 || best < p.splits)) p.live = 1;
+    else p.splits = best;
 }
 
 size_t vcpp_prefill_workspace_size(const vcpp_kv_pages* kv, int32_t num_chunks, int32_t max_chunk_len,

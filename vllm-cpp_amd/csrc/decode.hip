@@ -718,11 +718,12 @@ void decode_mfma_kernel(DecodeParams p) {
 // once, from a cold instruction cache): one tile per step, one buffer and one
 // masked form of it took 6.8 us for 128 tokens of 4 sequences (32/8 heads of
 // 128, fp16 pages) against 8.9 for the register kernel's four buffers and two
-// forms.  Four waves per SIMD hide the loads instead.
+// forms.  Its two workgroups per CU hide the loads instead (at 78 to 127 VGPRs,
+// the same with an occupancy target of two waves per SIMD).
 // Kernel plus merge against the page-staged kernel and its merge (us, fp16,
 // 32/8 heads of 128, uniform contexts of half the maximum and up): 4 x 128
 // 6.6 against 17.7, 4 x 1024 11.7 against 17.8, 16 x 1024 18.7 against 23.7,
-// 16 x 2048 28.4 against 33.4; the rule is plan_decode's.
+// 16 x 2048 28.4 against 33.4; the rule is small_partition's (api.cpp).
 // Rows that head slices do not cut at 128-byte lines were read 1.6 times
 // (head_dim 80) where a row's slices went to eight XCDs: a partition's slots on
 // one XCD take 32768 tokens (64/8 heads of 80) from 26.9 to 21.3 us, on int8
@@ -732,7 +733,7 @@ void decode_mfma_kernel(DecodeParams p) {
 constexpr int kSmallWaves = 4;
 constexpr int kXcds = 8;  // the dispatcher hands consecutive workgroups to consecutive XCDs
 // sp / num_seqs as a product with ceil(2^22 / num_seqs): exact for sp < 1024
-// (plan_decode's rule: two workgroups per CU).
+// (small_partition's rule: two workgroups per CU).
 constexpr int kSeqsShift = 22;
 
 template <int KV, int D>
@@ -813,16 +814,22 @@ void decode_small_kernel(DecodeParams p) {
 }
 
 // Tiles and non-empty sequences of the batch: all of them (T, K) and those
-// before s (S, KS), 64 sequences (one per lane) an add.
+// before s (S, KS), N sequences of each lane an add: i, i + 64, ..
 struct SplitSums {
     int T = 0, S = 0, K = 0, KS = 0;
+    template <int N>
     __device__ __forceinline__ void add(const DecodeParams& p, int s, int i) {
-        const int nt = i < p.num_seqs ? tiles_of(p, i) : 0;
-        const bool before = i < s;
-        T += wave_sum(nt);
-        S += wave_sum(before ? nt : 0);
-        K += __builtin_popcountll(__ballot(nt > 0));
-        KS += __builtin_popcountll(__ballot(before && nt > 0));
+        int nt[N];
+#pragma unroll
+        for (int k = 0; k < N; ++k) nt[k] = i + 64 * k < p.num_seqs ? tiles_of(p, i + 64 * k) : 0;
+#pragma unroll
+        for (int k = 0; k < N; ++k) {
+            const bool before = i + 64 * k < s;
+            T += wave_sum(nt[k]);
+            S += wave_sum(before ? nt[k] : 0);
+            K += __builtin_popcountll(__ballot(nt[k] > 0));
+            KS += __builtin_popcountll(__ballot(before && nt[k] > 0));
+        }
     }
 };
 
@@ -861,10 +868,7 @@ __global__ __launch_bounds__(FW * 64) void merge_split_kernel(DecodeParams p) {
     const int s = blockIdx.x;
     if (pair >= p.pairs) return;
     SplitSums c;
-    for (int base = 0; base < p.num_seqs; base += 128) {
-        c.add(p, s, base + lane);
-        c.add(p, s, base + 64 + lane);
-    }
+    for (int base = 0; base < p.num_seqs; base += 128) c.add<2>(p, s, base + lane);
     const int mine = tiles_of(p, s);
     if (mine <= 0) return;  // no tiles: zeroed by the decode kernel
     merge_split_unit<D, FW>(p, c, mine, s, pair, blockIdx.z >> 2, threadIdx.x >> 6, lane, part);
@@ -886,7 +890,7 @@ __global__ __launch_bounds__((8 * D + 255) / 256 * 64) void merge_split_slot_ker
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int s = blockIdx.x;
     SplitSums c;
-    for (int base = 64 * wave; base < p.num_seqs; base += 64 * U) c.add(p, s, base + lane);
+    for (int base = 64 * wave; base < p.num_seqs; base += 64 * U) c.add<1>(p, s, base + lane);
     const int mine = tiles_of(p, s);
     if (lane == 0) sums[wave] = make_int4(c.T, c.S, c.K, c.KS);
     __syncthreads();
@@ -1882,7 +1886,9 @@ hipError_t launch_mfma(const DecodeParams& p, hipStream_t stream) {
 // Measured (us, 1 / 2 / 8 waves): one 32768-token sequence, 24 units of 256
 // fragments, 34.1 / 18.2 / 7.9; 16 x 32768, 384 units of 16, 5.2 / 4.7 / 5.1;
 // 40 sequences of 100..5000, 640 units of 13, 6.6 / 5.8 / 7.1; 64 of
-// 128..4096, 1536 units of 4, 4.8 / 4.9 / 9.4.
+// 128..4096, 1536 units of 4, 4.8 / 4.9 / 9.4.  Decode and merge over 4568
+// drawn batches of up to 128 sequences: none over 1.2 % slower than with one
+// wave per 8 heads throughout.
 int merge_waves(int64_t units) { return units * 8 <= 2048 ? 8 : units * 2 <= 2048 ? 2 : 1; }
 
 template <int D, int FW>

@@ -104,7 +104,9 @@ typedef struct vcpp_kv_pages {
  *   context_lens [num_seqs] int32 on the device
  *   max_context_len  host-side upper bound of context_lens (sizes the grid;
  *                a larger context_len is an error the kernel cannot report:
- *                positions past max_context_len are not attended)
+ *                positions past max_context_len are not attended).  A bound
+ *                near the longest length is fastest: small batches (below)
+ *                size their partitions by it
  *   partition_size   0 (default): the tiles of all sequences are split
  *                evenly over the workgroups the GPU holds at once (fp16/int8/fp8;
  *                small batches: partitions of 64..1024 tokens, chosen so that

@@ -476,7 +476,9 @@ std::mutex g_dense_mu;  // the split's two launches: they share the scratch
 // parts or more, 1.5 MiB for two or three.  Measured (us, unsplit / split):
 // 64 pairs x 4096 keys of 128 88.7 / 50.9, 64 x 1024 of 80 18.8 / 16.1;
 // 128 x 1024 of 128 30.0 / 30.5 (not split).  A second round of at most half
-// the CUs is also worth splitting for: 320 x 4096 of 128 249.6 / 214.9.
+// the CUs is also worth splitting for: 320 x 4096 of 128 249.6 / 214.9.  (From
+// 342 pairs the scratch holds two parts of each: 352 x 4096 241.8 / 225.2, at
+// the line 384 x 2048 127.7 / 128.1 and x 8192 515.5 / 499.0.)
 int dense_parts(const DenseParams& p, int cus) {
     const int64_t pairs = (int64_t)p.batch * p.heads, bytes = (int64_t)p.kv_len * p.head_dim * 8;
     if (pairs > cus) return 2 * pairs <= 3 * (int64_t)cus && bytes >= (2 << 20) ? 3 : 1;

@@ -55,21 +55,34 @@ def parts(lens, prefixes, heads, kv_heads, dim, cus=256, caps=None):
     """Parts of chunks of these lengths; caps: (max_chunk_len, max_prefix_len)."""
     rows, prefix = caps or (max(lens), max(prefixes))
     most = most_parts(len(lens), rows, prefix, heads, kv_heads, dim, cus)
-    live = rows > tile_rows(dim)
-    if live and len(lens) == 1 and caps and parts([rows], [prefix], heads, kv_heads, dim, cus) == most:
-        return most  # one chunk's fullest count, by the host's bounds
-    if not live:
-        lens, prefixes = [rows] * len(lens), [prefix] * len(lens)
-    zh = kv_heads * -(-(heads // kv_heads) // 4)
-    items = sum(-(-n // tile_rows(dim)) for n in lens) * zh
+    if most == 1 or len(lens) > 64:
+        return most
+    by_bounds = least_cost([rows] * len(lens), [prefix] * len(lens), heads, kv_heads, dim, cus, most)
+    if not live(lens, by_bounds, most, rows, dim):
+        return by_bounds
     keys = max(n + p for n, p in zip(lens, prefixes) if n > 0)
+    return least_cost(lens, prefixes, heads, kv_heads, dim, cus, max(1, min(most, keys // 256)))
+
+
+def live(lens, by_bounds, most, rows, dim):
+    several = rows > tile_rows(dim)
+    return several or by_bounds < most if len(lens) > 1 else several and by_bounds < most
+
+
+def least_cost(lens, prefixes, heads, kv_heads, dim, cus, most):
+    zh = kv_heads * -(-(heads // kv_heads) // 4)
+    tiles = [-(-n // tile_rows(dim)) for n in lens]
+    items = sum(tiles) * zh
+    keys = max(n + p for n, p in zip(lens, prefixes) if n > 0)
+    work = sum(t * (n + p) for t, n, p in zip(tiles, lens, prefixes)) * zh
 
     def cost(s):
         full, rest = divmod(items * s, 2 * cus)
-        return (keys / (32 * s) * (full + (0 if rest == 0 else 0.72 if rest <= cus else 1)) + 5 * (full + (rest > 0)) +
-                (s * sum(lens) * heads * dim * 8 / 6.5e6 if s > 1 else 0))
+        part = keys / (32 * s)
+        return (min(part * (full + (0 if rest == 0 else 0.72 if rest <= cus else 1)), work / (64 * cus) + part / 2) +
+                5 * (full + (rest > 0)) + (s * sum(lens) * heads * dim * 8 / 6.5e6 if s > 1 else 0))
 
-    return min((s for s in range(1, most + 1) if s == 1 or not live or s * 512 <= keys), key=cost)
+    return min(range(1, most + 1), key=cost)
 
 
 # (row counts, prefixes, heads, kv heads, head_dim)
@@ -95,16 +108,18 @@ def test_one_chunk_loose_bounds():
     assert parts([90], [200], 64, 8, 80, caps=(300, 16384)) == 1
 
 
-def test_one_tile_a_chunk():
-    """The host's choice where a chunk has one tile at most: never more than
-    the fullest count, and the restated rule's."""
-    for chunks in (1, 2, 5, 20):
-        for rows in (1, 31, 32, 33, 64):
+def test_workspace_asked():
+    """A call asks for its own count's workspace where the host chose it, for
+    the fullest count's where the device does."""
+    for chunks in (1, 2, 5, 20, 65):
+        for rows in (1, 31, 33, 64, 200):
             for prefix in (0, 700, 5000, 40000):
-                for heads, kv_heads, dim in ((64, 8, 80), (28, 4, 128), (8, 8, 64)):
-                    if rows > tile_rows(dim):
-                        continue
+                for heads, kv_heads, dim in ((64, 8, 80), (28, 4, 128), (8, 8, 64), (1, 1, 64)):
+                    most = most_parts(chunks, rows, prefix, heads, kv_heads, dim)
                     s = parts([rows] * chunks, [prefix] * chunks, heads, kv_heads, dim)
+                    if most > 1 and chunks <= 64:
+                        bounds = least_cost([rows] * chunks, [prefix] * chunks, heads, kv_heads, dim, 256, most)
+                        s = most if live([rows] * chunks, bounds, most, rows, dim) else s
                     assert need(chunks, rows, prefix, heads, kv_heads, dim) == bytes_of(s, chunks, rows, heads, dim)
 
 

@@ -145,17 +145,17 @@ def test_chunk_longer_than_max_chunk_len(cuda, split):
     ([33, 0, 1], [1000, 0, 5], 8, 1, 128, None),        # an empty chunk
     ([90], [200], 64, 8, 80, (300, 9000)),              # the real keys are too few to cut: finished in place
     ([90], [200], 64, 8, 80, (90, 9000)),               # one chunk's fullest count, more parts than key blocks
-    ([20, 9, 31], [3000, 800, 1700], 32, 8, 128, None), # one tile a chunk: the host's count
+    ([20, 9, 31], [3000, 800, 1700], 32, 8, 128, None), # one tile a chunk
+    ([20, 9, 31, 30] * 5, [3000, 800, 1700, 900] * 5, 12, 2, 128, None),  # and uneven prefixes, fewer than the fullest
     ([33] * 65, [1100] * 65, 1, 1, 128, None)])          # more chunks than lanes: the fullest count
 def test_parts_by_real_lengths(cuda, lens, prefixes, H, Hkv, D, caps):
     """The count the workgroups and the merge choose by the device's lengths is
     the restated rule's: parts past it leave their workspace as it was."""
-    from test_prefill_parts import most_parts, parts
+    from test_prefill_parts import least_cost, live, most_parts, parts
     rows, prefix = caps or (max(lens), max(prefixes))
     cus = torch.cuda.get_device_properties(0).multi_processor_count
     most = most_parts(len(lens), rows, prefix, H, Hkv, D, cus)
-    host = parts(lens, prefixes, H, Hkv, D, cus, caps)
-    want_parts = most if len(lens) > 64 else host
+    want_parts = parts(lens, prefixes, H, Hkv, D, cus, caps)
     assert most > 1
     pool, q16, q32, tables, q_start, pre = make_case(O.ORC_F16, 760 + D, prefixes, lens, H, Hkv, D)
     want = O.prefill(pool, q32, tables, q_start, pre, H)
@@ -167,8 +167,9 @@ def test_parts_by_real_lengths(cuda, lens, prefixes, H, Hkv, D, caps):
                                workspace=ws.view(torch.uint8))
     torch.cuda.synchronize()
     assert_close(out.cpu().numpy(), want, ATOL, RTOL, what="split parts %s" % (lens,))
-    if rows <= 32:
-        return  # (test_prefill_parts.py)
+    bounds = least_cost([rows] * len(lens), [prefix] * len(lens), H, Hkv, D, cus, most)
+    if len(lens) <= 64 and bounds < most and not live(lens, bounds, most, rows, D):
+        return  # the workspace holds that count's partials only (test_prefill_parts.py)
     slab = len(lens) * rows * H * D  # of one part's outputs, first row of the first chunk in its head
     written = [s for s in range(most) if not torch.isnan(ws[s * slab])]
     assert written == (list(range(want_parts)) if want_parts > 1 else [])

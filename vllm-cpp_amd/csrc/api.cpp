@@ -656,11 +656,12 @@ static int32_t prefill_most_splits(const vcpp_kv_pages* kv, int32_t num_chunks, 
     return (int32_t)std::max<int64_t>(1, std::min<int64_t>({want, by_len, (int64_t)vcpp::kMaxPrefillSplits}));
 }
 
-// Key parts of a split call.  The count of least cost by the host's bounds is
-// the call's where they say it all (one tile to a chunk) or where it is one
-// chunk's fullest count anyway; otherwise up to prefill_most_splits by the
-// lengths the device holds (`live`, the workgroups' choice, about 1.5 us of a
-// 380 us call).  More than 64 chunks (and the wide kernel): the fullest count.
+// Key parts of a split call.  By the host's bounds the count of least cost,
+// where that is the fullest one anyway or the bounds say it all (one chunk of
+// one tile); otherwise, and wherever chunks of several tiles can be uneven, up
+// to prefill_most_splits by the lengths the device holds (`live`, the
+// workgroups' choice, about 1.5 us of a 380 us call).  More than 64 chunks (and
+// the wide kernel): the fullest count.
 static void choose_splits(vcpp::PrefillParams& p, const vcpp_kv_pages* kv, int32_t max_prefix_len) {
     p.splits = prefill_most_splits(kv, p.num_chunks, p.max_chunk_len, max_prefix_len, p.num_heads);
     if (p.splits == 1 || p.num_chunks > 64 || vcpp::prefill_uses_wide(kv->dtype, kv->head_dim, kv->block_size)) return;
@@ -668,13 +669,13 @@ static void choose_splits(vcpp::PrefillParams& p, const vcpp_kv_pages* kv, int32
     const float keys = (float)max_prefix_len + p.max_chunk_len;
     const float out_values = (float)p.num_chunks * p.max_chunk_len * p.num_heads * kv->head_dim;
     const auto cost = [&](int32_t s) {
-        return vcpp::prefill_split_cost(s, items, items * s / (2 * cus), keys, out_values, cus);
+        return vcpp::prefill_split_cost(s, items, items * s / (2 * cus), keys, items * keys, out_values, cus);
     };
     int32_t best = 1;
     for (int32_t s = 2; s <= p.splits; ++s)
         if (cost(s) < cost(best)) best = s;
     const bool several = p.max_chunk_len > vcpp::prefill_tile_rows(kv->dtype, kv->head_dim, kv->block_size);
-    if (several && (p.num_chunks > 1 || best < p.splits)) p.live = 1;
+    if (p.num_chunks > 1 ? several || best < p.splits : several && best < p.splits) p.live = 1;
     else p.splits = best;
 }
 

@@ -53,21 +53,27 @@ struct PrefillParams {
 };
 
 // Cost of a split call in s key parts, of `items` workgroups a part whose
-// longest keys are `keys`, in units of one 32-key block of two resident
-// workgroups per CU (about 1.3 us): a round of a part's blocks, 0.72 of that
-// where the last round leaves one workgroup per CU, 5 for a round's start and
-// end, and the partials' traffic.  The fullest count is not the best where it
-// spills a few workgroups into a round of their own: 48 tiles in 11 parts are
-// 528 workgroups, 56.0 us for three 40-token chunks on 7000-token prefixes
-// (32/8 heads of 128), 41.9 in 10 parts; but 384 tiles (three 500-token chunks
-// on 8192, 64/8 heads of 80) take 365 us whole and 325 in two parts.  Over 3746
-// drawn calls, each timed at every count, the count of least cost takes 1.0015
-// of the best one's time in the geometric mean, 0.952 of the fullest one's.
+// longest keys are `keys` and whose keys sum to `work`, in units of one 32-key
+// block of two resident workgroups per CU (about 1.3 us): a round of a part's
+// blocks, 0.72 of that where the last round leaves one workgroup per CU, or
+// (uneven prefixes) the blocks spread evenly and half the longest part's after
+// them; 5 for a round's start and end, and the partials' traffic.  The fullest
+// count is not the best where it spills a few workgroups into a round of their
+// own: 48 tiles in 11 parts are 528 workgroups, 56.0 us for three 40-token
+// chunks on 7000-token prefixes (32/8 heads of 128), 41.9 in 10 parts; but 384
+// tiles (three 500-token chunks on 8192, 64/8 heads of 80) take 365 us whole
+// and 325 in two parts.  Every count of drawn calls was timed: over 3746 calls
+// of up to 3 chunks the count of least cost takes 1.0015 of the best one's time
+// in the geometric mean (the fullest one 1.038), over 5286 of 4 to 64 chunks
+// 1.003 (1.026; by rounds of the longest keys alone 1.0065).
 // (full: items * s / (2 * cus), whole rounds.)
-__host__ __device__ inline float prefill_split_cost(int s, int items, int full, float keys, float out_values, int cus) {
-    const int rest = items * s - full * 2 * cus;
-    return keys / (32.f * s) * (full + (rest == 0 ? 0.f : rest <= cus ? 0.72f : 1.f)) + 5.f * (full + (rest > 0)) +
-           (s > 1 ? s * out_values * (8.f / 6.5e6f) : 0.f);
+__host__ __device__ inline float prefill_split_cost(int s, int items, int full, float keys, float work,
+                                                    float out_values, int cus) {
+    const int slots = 2 * cus, rest = items * s - full * slots;
+    const float part = keys / (32.f * s);
+    const float rounds = part * (full + (rest == 0 ? 0.f : rest <= cus ? 0.72f : 1.f));
+    const float even = work / (32.f * slots) + 0.5f * part;
+    return (rounds < even ? rounds : even) + 5.f * (full + (rest > 0)) + (s > 1 ? s * out_values * (8.f / 6.5e6f) : 0.f);
 }
 
 hipError_t launch_prefill(const PrefillParams& p, hipStream_t stream);

@@ -142,21 +142,23 @@ __device__ __forceinline__ int div_small(int a, int b) {
 }
 
 // Key parts of a split call by the chunks' real lengths: of 1 .. p.splits the
-// count of least cost, at least 512 keys of the longest chunk to a part.  By
+// count of least cost, at least 256 keys of the longest chunk to a part.  By
 // max_chunk_len the host would count tiles that short chunks do not have, and
 // so take too few parts (three chunks of 178..449 rows on prefixes up to 19757,
 // 24/8 heads of 80: 432 us in two parts, 301 in three).  Lane s - 1 weighs s
 // parts, and every workgroup and the merge come to the same count.
 __device__ __forceinline__ int live_splits(const PrefillParams& p, const LiveChunks& c, int lane) {
     const int keys = wave_max0(c.tiles > 0 ? c.prefix + c.n : 0);
+    const float work = (float)wave_sum(c.tiles * (c.prefix + c.n)) * (p.num_kv_heads * p.head_groups);
     const int last = p.num_chunks - 1;
     const int rows = __builtin_amdgcn_readlane(c.q0 + c.n, last) - __builtin_amdgcn_readlane(c.q0, 0);
     const float out_values = (float)rows * (p.num_heads * p.head_dim);
     const int items = c.total * p.num_kv_heads * p.head_groups, cus = max(8 * p.xcd_cus, 1);
     const int s = lane + 1;
     uint32_t best = ~0u;  // cost (positive: its bits are ordered), low bits the count
-    if (s <= p.splits && (s == 1 || s * 512 <= keys)) {
-        const float cost = prefill_split_cost(s, items, div_small(items * s, 2 * cus), (float)keys, out_values, cus);
+    if (s <= p.splits && (s == 1 || s * 256 <= keys)) {
+        const float cost = prefill_split_cost(s, items, div_small(items * s, 2 * cus), (float)keys, work,
+                                              out_values, cus);
         best = ((uint32_t)__float_as_int(cost) & ~15u) | lane;
     }
     static_assert(kMaxPrefillSplits == 16, "counts in four bits, of one row of lanes");
